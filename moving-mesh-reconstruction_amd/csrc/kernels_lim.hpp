@@ -1,4 +1,4 @@
-// kernels_lim.hpp -- grid limiter (calcdefp), relaxing-TVD transport and FFT kernels.
+// kernels_lim.hpp -- grid limiter (calcdefp), and relaxing-TVD transport kernels.
 // Same conventions as kernels.hpp: column-major, periodic, reference association order,
 // built with -ffp-contract=off.
 #pragma once
@@ -195,142 +195,23 @@ __global__ __launch_bounds__(256) void k_complim(T* __restrict__ lim, const T* _
   if (threadIdx.x == 0) { bstat[2 * (i64)blockIdx.x] = s[0][0]; bstat[2 * (i64)blockIdx.x + 1] = s[1][0]; }
 }
 
-template <class T> __global__ void k_axpy_scale(T* __restrict__ y, const T* __restrict__ x, int n, i64 n3) {
-  // y += ((x*2)/n/n/n)  (mmh/limiter.f90:579,592)
+// The compression limiter's correction x (its inverse transform, unnormalised): v = x 2 / n / n / n
+// (mmh/limiter.f90:579,592) is added to defp and stored in tmp2, leading dimension n + 2
+// (limiter.f90:43).  1 / n is exact (n a power of two), so each product rounds as the division does.
+template <class T>
+__global__ void k_limit_apply(T* __restrict__ defp, T* __restrict__ tmp2, const T* __restrict__ x, int n, i64 n3) {
   const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n3) return;
-  T v = x[p] * T(2.) / T(n) / T(n) / T(n);
-  y[p] = y[p] + v;
+  const T rn = T(1) / T(n);
+  const T v = x[p] * T(2.) * rn * rn * rn;
+  defp[p] = defp[p] + v;
+  const i64 i = p & (n - 1), r = p >> __builtin_ctz(n);
+  tmp2[i + (i64)(n + 2) * r] = v;
 }
 
 template <class T> __global__ void k_add(T* __restrict__ y, const T* __restrict__ x, i64 n3) {
   const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (p < n3) y[p] = y[p] + x[p];
-}
-
-// ------------------------------------------------------------------------------------------------
-// FFT: radix-2 Stockham per line in LDS.  One workgroup per line; twiddles W[q] = exp(s*2*pi*i*q/L)
-// come from a host table so that rounding matches the CPU restatement exactly.
-template <class T> struct C2 { T r, i; };
-
-template <class T>
-__global__ void k_fft_lines(C2<T>* __restrict__ z, const C2<T>* __restrict__ W, int L, int d0, int d1, int axis) {
-  extern __shared__ unsigned char smem_raw[];
-  C2<T>* a = reinterpret_cast<C2<T>*>(smem_raw);
-  C2<T>* b = a + L;
-  const i64 l = blockIdx.x;
-  i64 base, st;
-  if (axis == 0) { base = l * (i64)d0; st = 1; }
-  else if (axis == 1) { base = (l % d0) + (l / d0) * (i64)d0 * d1; st = d0; }
-  else { base = l; st = (i64)d0 * d1; }
-  for (int q = threadIdx.x; q < L; q += blockDim.x) a[q] = z[base + q * st];
-  __syncthreads();
-  int p = 1;
-  while (p < L) {
-    const int stride = L / (2 * p);
-    for (int i = threadIdx.x; i < L / 2; i += blockDim.x) {
-      const int k = i & (p - 1);
-      const C2<T> w = W[k * stride];
-      const C2<T> u0 = a[i], u1 = a[i + L / 2];
-      T tr = w.r * u1.r - w.i * u1.i;
-      T ti = w.r * u1.i + w.i * u1.r;
-      const int jj = 2 * i - k;
-      b[jj].r = u0.r + tr; b[jj].i = u0.i + ti;
-      b[jj + p].r = u0.r - tr; b[jj + p].i = u0.i - ti;
-    }
-    __syncthreads();
-    C2<T>* t = a; a = b; b = t;
-    p <<= 1;
-  }
-  for (int q = threadIdx.x; q < L; q += blockDim.x) z[base + q * st] = a[q];
-}
-
-// rlft3 recombination between the half-length complex transform and the real spectrum
-// (mmh/recipes12.f90:100-127).  Pass A handles k1 = 0 with the Nyquist plane speq (needs the
-// previous speq, sold); pass B the pairs (i1, n1/2 - i1), 1 <= i1 < n1/4.
-template <class T>
-__global__ void k_rlft_k0(C2<T>* __restrict__ z, C2<T>* __restrict__ sq, const C2<T>* __restrict__ sold, int h1, int n2, int n3,
-                          T c2i) {
-  const i64 q = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (i64)n2 * n3) return;
-  const int i2 = (int)(q % n2), i3 = (int)(q / n2);
-  const int j2 = i2 == 0 ? 0 : n2 - i2, j3 = i3 == 0 ? 0 : n3 - i3;
-  C2<T> X = z[(i64)h1 * ((i64)i2 + (i64)n2 * i3)], Y = sold[j2 + (i64)n2 * j3];
-  C2<T> s{X.r + Y.r, X.i - Y.i}, d{X.r - Y.r, X.i + Y.i};
-  C2<T> H1{T(0.5) * s.r, T(0.5) * s.i};
-  C2<T> H2{-c2i * d.i, c2i * d.r};
-  z[(i64)h1 * ((i64)i2 + (i64)n2 * i3)] = C2<T>{H1.r + H2.r, H1.i + H2.i};
-  sq[j2 + (i64)n2 * j3] = C2<T>{H1.r - H2.r, -(H1.i - H2.i)};
-}
-
-template <class T>
-__global__ void k_rlft_pairs(C2<T>* __restrict__ z, const C2<T>* __restrict__ wtab, int h1, int n2, int n3, T c2i) {
-  // one thread per (i1, i2, i3) with 1 <= i1 < h1 - i1
-  const int npair = (h1 - 1) / 2;  // number of i1 values with i1 < h1 - i1, i1 >= 1
-  const i64 q = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (i64)npair * n2 * n3) return;
-  const int i1 = 1 + (int)(q % npair);
-  const i64 r = q / npair;
-  const int i2 = (int)(r % n2), i3 = (int)(r / n2);
-  const int j1 = h1 - i1, j2 = i2 == 0 ? 0 : n2 - i2, j3 = i3 == 0 ? 0 : n3 - i3;
-  const T wr = wtab[i1].r, wi = wtab[i1].i;
-  C2<T>& Xr = z[(i64)i1 + (i64)h1 * ((i64)i2 + (i64)n2 * i3)];
-  C2<T>& Yr = z[(i64)j1 + (i64)h1 * ((i64)j2 + (i64)n2 * j3)];
-  C2<T> X = Xr, Y = Yr;
-  C2<T> s{X.r + Y.r, X.i - Y.i}, d{X.r - Y.r, X.i + Y.i};
-  C2<T> H1{T(0.5) * s.r, T(0.5) * s.i};
-  C2<T> H2{-c2i * d.i, c2i * d.r};
-  C2<T> WH{wr * H2.r - wi * H2.i, wr * H2.i + wi * H2.r};
-  Xr = C2<T>{H1.r + WH.r, H1.i + WH.i};
-  Yr = C2<T>{H1.r - WH.r, -(H1.i - WH.i)};
-}
-
-// Spectral operations on the rlft3 layout: data (n x n x n reals = complex h x n x n) + speq (n x n).
-// mode 0: divide by the 7-point symbol 2cos kx + 2cos ky + 2cos kz - 6 (mmh/limiter.f90:560-575)
-// from host cosine tables; mode 1: multiply by |k|^2 (mmh/reconstruct.f90:14-36);
-// mode 2/3/4: multiply by i k_x, i k_y, i k_z (mmh/gradient.f90:16-26, 34-48, 56-70).
-template <class T>
-__global__ void k_spectral(T* __restrict__ data, T* __restrict__ speq, int n, int mode, const T* __restrict__ cosx,
-                           const T* __restrict__ cosy, const T* __restrict__ cosz, T pi) {
-  const int h = n / 2;
-  const i64 q = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (i64)(h + 1) * n * n) return;
-  const int ic = (int)(q % (h + 1));
-  const i64 r = q / (h + 1);
-  const int j = (int)(r % n), k = (int)(r / n);
-  T* re = ic < h ? &data[ix3(2 * ic, j, k, n)] : &speq[2 * ((i64)j + (i64)n * k)];
-  if (mode == 0) {
-    T ak = T(2) * cosx[ic] + T(2) * cosy[j] + T(2) * cosz[k] - T(6);
-    if (fabs(ak) < T(1e-10)) ak = 1;
-    re[0] = re[0] / ak;
-    re[1] = re[1] / ak;
-  } else if (mode == 1) {
-    T k3 = (k + 1 <= h + 1) ? T(k) : T(k - n);
-    k3 = k3 / T(n) * T(2.) * pi;
-    T k2 = (j + 1 <= h + 1) ? T(j) : T(j - n);
-    k2 = k2 / T(n) * T(2.) * pi;
-    T k1 = T(ic);
-    k1 = k1 / T(n) * T(2.) * pi;
-    T f = k1 * k1 + k2 * k2 + k3 * k3;
-    re[0] = re[0] * f;
-    re[1] = re[1] * f;
-  } else {
-    T km;
-    if (mode == 2) km = T(ic);
-    else if (mode == 3) km = (j + 1 <= h + 1) ? T(j) : T(j - n);
-    else km = (k + 1 <= h + 1) ? T(k) : T(k - n);
-    T A = re[0], Bv = re[1];
-    T cr = A * T(0) - Bv * km, ci = A * km + Bv * T(0);
-    cr = cr / T(n) * T(2.) * pi;
-    ci = ci / T(n) * T(2.) * pi;
-    re[0] = cr;
-    re[1] = ci;
-  }
-}
-
-template <class T> __global__ void k_scale2(T* __restrict__ out, const T* __restrict__ in, int n, i64 n3) {
-  const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < n3) out[p] = in[p] * T(2.) / T(n) / T(n) / T(n);
 }
 
 // ------------------------------------------------------------------------------------------------

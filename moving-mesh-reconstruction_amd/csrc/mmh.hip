@@ -22,6 +22,7 @@
 
 #include "../../include/mmh.h"
 #include "kernels.hpp"
+#include "kernels_fft.hpp"
 #include "kernels_lim.hpp"
 #include "kernels_adj.hpp"
 #include "kernels_wave.hpp"
@@ -841,72 +842,115 @@ template <class T> const C2<T>* twiddle_table(mmh_ctx* c, int L, int s) {
   return d;
 }
 
-template <class T> void fft3_dev(mmh_ctx* c, C2<T>* z, int d0, int d1, int d2, int s) {
-  const int dims[3] = {d0, d1, d2};
-  for (int ax = 0; ax < 3; ++ax) {
-    const int L = dims[ax];
-    if (L == 1) continue;
-    const C2<T>* W = twiddle_table<T>(c, L, s);
-    const i64 nl = (i64)d0 * d1 * d2 / L;
-    const int thr = std::max(64, std::min(256, L / 2));
-    k_fft_lines<T><<<(unsigned)nl, thr, 2 * L * sizeof(C2<T>), c->stream>>>(z, W, L, d0, d1, ax);
-    LAUNCHCHK();
+// f(integral_constant<int, L>) for the line length L, a power of two from 2 to 2048 (longer lines
+// would belong to arrays that no device holds).
+template <class F> void for_line(int L, F&& f) {
+  switch (L) {
+    case 2: return f(std::integral_constant<int, 2>());
+    case 4: return f(std::integral_constant<int, 4>());
+    case 8: return f(std::integral_constant<int, 8>());
+    case 16: return f(std::integral_constant<int, 16>());
+    case 32: return f(std::integral_constant<int, 32>());
+    case 64: return f(std::integral_constant<int, 64>());
+    case 128: return f(std::integral_constant<int, 128>());
+    case 256: return f(std::integral_constant<int, 256>());
+    case 512: return f(std::integral_constant<int, 512>());
+    case 1024: return f(std::integral_constant<int, 1024>());
+    case 2048: return f(std::integral_constant<int, 2048>());
   }
+  throw MmhError(MMH_ENOMEM, "fft: lines longer than 2048 do not fit in device memory as a cube");
 }
 
-template <class T> __global__ void k_get_speq(C2<T>* sq, const C2<T>* z, int h1, i64 m) {
-  const i64 q = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < m) sq[q] = z[(i64)h1 * q];
+template <class T> void fft_x(mmh_ctx* c, C2<T>* out, const C2<T>* in, int d0, i64 nl, int s) {
+  const C2<T>* W = twiddle_table<T>(c, d0, s);
+  for_line(d0, [&](auto len) {
+    constexpr int L = decltype(len)::value, NL = 256 / FftShape<L>::TL;
+    k_fft_x<T, L><<<(unsigned)((nl + NL - 1) / NL), 256, 0, c->stream>>>(out, in, W, nl);
+  });
+  LAUNCHCHK();
+}
+// Lines of length d and stride inner (axis 1: inner = d0; axis 2: inner = d0 d1); scale as in k_fft_cols.
+template <class T>
+void fft_cols(mmh_ctx* c, C2<T>* out, const C2<T>* in, int d, i64 inner, i64 total, int s, T scale = T(0)) {
+  const C2<T>* W = twiddle_table<T>(c, d, s);
+  const i64 nl = total / d;
+  const int lgi = __builtin_ctzll((unsigned long long)inner);
+  for_line(d, [&](auto len) {
+    constexpr int L = decltype(len)::value;
+    using K = FftCols<T, L>;
+    k_fft_cols<T, L><<<(unsigned)((nl + K::C - 1) / K::C), K::NT, 0, c->stream>>>(out, in, W, nl, lgi, scale);
+  });
+  LAUNCHCHK();
 }
 
-template <class T> void rlft3_dev(mmh_ctx* c, T* data, T* speq, int n, int isign) {
+// Complex transform over all three axes (out may equal in); scale: the inverse's normalisation.
+template <class T> void fft3_dev(mmh_ctx* c, C2<T>* out, const C2<T>* in, int d0, int d1, int d2, int s, T scale = T(0)) {
+  const i64 total = (i64)d0 * d1 * d2;
+  fft_x<T>(c, out, in, d0, total / d0, s);
+  fft_cols<T>(c, out, out, d1, d0, total, s);
+  fft_cols<T>(c, out, out, d2, (i64)d0 * d1, total, s, scale);
+}
+
+// rlft3 by itself: forward from the field `in` (may equal data) into (data, speq); inverse of (data,
+// speq) into out (null: data), normalised when scale > 0.
+template <class T>
+void rlft3_dev(mmh_ctx* c, T* data, const T* in, T* speq, int n, int isign, T* out = nullptr, T scale = T(0)) {
   C2<T>* z = reinterpret_cast<C2<T>*>(data);
   C2<T>* sq = reinterpret_cast<C2<T>*>(speq);
   const int h1 = n / 2;
   const i64 m = (i64)n * n;
-  if (isign == 1) {
-    fft3_dev<T>(c, z, h1, n, n, 1);
-    k_get_speq<T><<<nblk(m), 256, 0, c->stream>>>(sq, z, h1, m);
-    LAUNCHCHK();
-  }
-  C2<T>* sold = wsT<C2<T>>(c, "rlft_sold", m);
-  HIPCHK(hipMemcpyAsync(sold, sq, sizeof(C2<T>) * m, hipMemcpyDeviceToDevice, c->stream));
+  if (isign == 1) fft3_dev<T>(c, z, reinterpret_cast<const C2<T>*>(in), h1, n, n, 1);
   const T c2i = T(-0.5) * T(isign);
-  k_rlft_k0<T><<<nblk(m), 256, 0, c->stream>>>(z, sq, sold, h1, n, n, c2i);
+  k_rlft_k0<T><<<nblk(m), 256, 0, c->stream>>>(z, sq, h1, n, isign == 1 ? 1 : 0, c2i);
   LAUNCHCHK();
   const int npair = (h1 - 1) / 2;
   if (npair > 0) {
-    std::vector<C2<T>> w(h1);
-    for (int i1 = 0; i1 < h1; ++i1) {
-      double ang = 2.0 * M_PI * (double)i1 / (double)n;
-      w[i1].r = (T)cos(ang);
-      w[i1].i = (T)((double)isign * sin(ang));
-    }
-    C2<T>* wd = wsT<C2<T>>(c, std::string("rlft_w") + (isign > 0 ? "p" : "m") + std::to_string(n), h1);
-    HIPCHK(hipMemcpyAsync(wd, w.data(), sizeof(C2<T>) * h1, hipMemcpyHostToDevice, c->stream));
-    k_rlft_pairs<T><<<nblk((i64)npair * m), 256, 0, c->stream>>>(z, wd, h1, n, n, c2i);
+    k_rlft_pairs<T><<<nblk((i64)npair * m), 256, 0, c->stream>>>(z, twiddle_table<T>(c, n, isign), h1, n, n, c2i);
     LAUNCHCHK();
-    HIPCHK(hipStreamSynchronize(c->stream));
   }
-  if (isign == -1) fft3_dev<T>(c, z, h1, n, n, -1);
+  if (isign == -1) fft3_dev<T>(c, reinterpret_cast<C2<T>*>(out ? out : data), z, h1, n, n, -1, scale);
 }
 
-// Spectral multiplier pass on (data, speq); mode as in k_spectral.
-template <class T> void spectral(mmh_ctx* c, T* data, T* speq, int n, int mode) {
+// Cosine tables of spectral_mul's mode 0, uploaded once per size.
+template <class T> const T* cosine_table(mmh_ctx* c, int n) {
   const T pi2 = T(3.14159265358979323846264338328);      // limiter.f90:59
-  const T piG = (T)(atan(1.0) * 4.0);                   // gradient.f90:10, reconstruct.f90:9
-  T* cs = wsT<T>(c, "spec_cos" + std::to_string(n), 3 * (i64)n);
-  if (mode == 0) {
+  const std::string key = "spec_cos" + std::to_string(n), ukey = key + ":" + std::to_string(sizeof(T));
+  T* cs = wsT<T>(c, key, 3 * (i64)n);
+  if (!c->uploaded.count(ukey)) {
     std::vector<T> h(3 * (size_t)n);
     for (int ii = 0; ii <= n / 2; ++ii) h[ii] = (T)std::cos((T)(T(2) * pi2 * T(ii) / T(n)));
     for (int j = 0; j < n; ++j) h[n + j] = (T)std::cos((T)(T(2) * pi2 * (T(j + 1) - T(1.)) / T(n)));
     for (int k = 0; k < n; ++k) h[2 * n + k] = h[n + k];
     HIPCHK(hipMemcpyAsync(cs, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    c->uploaded.insert(ukey);
   }
-  const i64 cnt = (i64)(n / 2 + 1) * n * n;
-  k_spectral<T><<<nblk(cnt), 256, 0, c->stream>>>(data, speq, n, mode, cs, cs + n, cs + 2 * n, piG);
+  return cs;
+}
+
+// out = inverse transform of the multiplier `mode` times the spectrum whose forward complex
+// transform (three axes, not yet recombined) is `spec` (may equal out): the middle of the operation
+// and the inverse x lines in one pass, then the y and z axes.  speq (may be null): the Nyquist
+// plane as rlft3 leaves it.
+template <class T>
+void spectral_inverse(mmh_ctx* c, T* out, const T* spec, T* speq, int n, int mode, int zero_dc, T scale) {
+  const T piG = (T)(atan(1.0) * 4.0);                   // gradient.f90:10, reconstruct.f90:9
+  const T* cs = mode == 0 ? cosine_table<T>(c, n) : nullptr;
+  const C2<T>* Wp = twiddle_table<T>(c, n, 1);
+  const C2<T>* Wm = twiddle_table<T>(c, n, -1);
+  const C2<T>* W = twiddle_table<T>(c, n / 2, -1);
+  C2<T>* z = reinterpret_cast<C2<T>*>(out);
+  const i64 total = cube(n) / 2;
+  for_line(n / 2, [&](auto len) {
+    constexpr int L = std::min(decltype(len)::value, 1024), NP = 128 / FftShape<L>::TL;
+    require(2 * L == n, "spectral: n up to 2048");
+    const i64 pairs = (i64)(L - 1) * n + 2 * (L + 1);
+    k_rlft_mid<T, L><<<(unsigned)((pairs + NP - 1) / NP), 256, 0, c->stream>>>(
+        z, reinterpret_cast<const C2<T>*>(spec), Wp, Wm, W, reinterpret_cast<C2<T>*>(speq), mode, zero_dc, cs, piG);
+  });
   LAUNCHCHK();
+  fft_cols<T>(c, z, z, n, n / 2, total, -1);
+  fft_cols<T>(c, z, z, n, (i64)n * n / 2, total, -1, scale);
 }
 
 template <class T> void nsmooth_dev(mmh_ctx* c, T* a, int n, int times) {
@@ -1012,21 +1056,17 @@ void calcdefp_dev(mmh_ctx* c, T* defp, T* tmp, T* tmp2, const T* def, const T* u
   long ncompress = 0;
   double cmax = 0;
   for (unsigned b = 0; b < nb; ++b) { ncompress += (long)hb2[2 * b]; cmax = std::max(cmax, hb2[2 * b + 1]); }
-  k_pad<T><<<nblk(n3), 256, 0, c->stream>>>(tmp2, lim, n, n3);
-  LAUNCHCHK();
   if (ncompress > 0) {
     T* sq = wsT<T>(c, "limS", 2 * (i64)n * n);
-    fill<T>(c, sq, T(0), 2 * (i64)n * n);
-    rlft3_dev<T>(c, lim, sq, n, 1);
-    spectral<T>(c, lim, sq, n, 0);
-    fill<T>(c, lim, T(0), 1);
-    rlft3_dev<T>(c, lim, sq, n, -1);
-    k_axpy_scale<T><<<nblk(n3), 256, 0, c->stream>>>(defp, lim, n, n3);
-    k_scale2<T><<<nblk(n3), 256, 0, c->stream>>>(lim, lim, n, n3);
-    k_pad<T><<<nblk(n3), 256, 0, c->stream>>>(tmp2, lim, n, n3);
+    C2<T>* z = reinterpret_cast<C2<T>*>(lim);
+    fft3_dev<T>(c, z, z, n / 2, n, n, 1);
+    spectral_inverse<T>(c, lim, lim, sq, n, 0, 1, T(0));
+    k_limit_apply<T><<<nblk(n3), 256, 0, c->stream>>>(defp, tmp2, lim, n, n3);
     k_pad_speq<T><<<nblk((i64)n * n), 256, 0, c->stream>>>(tmp2, sq, n);
-    LAUNCHCHK();
+  } else {
+    k_pad<T><<<nblk(n3), 256, 0, c->stream>>>(tmp2, lim, n, n3);
   }
+  LAUNCHCHK();
   // exit convention of tmp (limiter.f90:621-628,669-671): all cells "hot" -> 1; diagnostics 0
   fill<T>(c, tmp, T(1), n3);
   fill<T>(c, tmp, T(0), 3);
@@ -1104,16 +1144,16 @@ void reconstruct_dev(mmh_ctx* c, T* u, T* def, T* defp, int n, int nf, int niter
 }
 
 template <class T> void spectral_out(mmh_ctx* c, const T* phi, T* out, int n, int mode) {
-  const i64 n3 = cube(n);
-  T* d = wsT<T>(c, "specD", n3);
-  T* sq = wsT<T>(c, "specS", 2 * (i64)n * n);
-  HIPCHK(hipMemcpyAsync(d, phi, sizeof(T) * n3, hipMemcpyDeviceToDevice, c->stream));
-  fill<T>(c, sq, T(0), 2 * (i64)n * n);
-  rlft3_dev<T>(c, d, sq, n, 1);
-  spectral<T>(c, d, sq, n, mode);
-  rlft3_dev<T>(c, d, sq, n, -1);
-  k_scale2<T><<<nblk(n3), 256, 0, c->stream>>>(out, d, n, n3);
-  LAUNCHCHK();
+  T* d = wsT<T>(c, "specD", cube(n));
+  fft3_dev<T>(c, reinterpret_cast<C2<T>*>(d), reinterpret_cast<const C2<T>*>(phi), n / 2, n, n, 1);
+  spectral_inverse<T>(c, out, d, nullptr, n, mode, 0, T(1) / T(n));
+}
+
+// scalar2gradient: the three components from one forward transform.
+template <class T> void gradient_dev(mmh_ctx* c, const T* phi, T* psi, int n) {
+  T* d = wsT<T>(c, "specD", cube(n));
+  fft3_dev<T>(c, reinterpret_cast<C2<T>*>(d), reinterpret_cast<const C2<T>*>(phi), n / 2, n, n, 1);
+  for (int a = 0; a < 3; ++a) spectral_inverse<T>(c, psi + (i64)a * cube(n), d, nullptr, n, 2 + a, 0, T(1) / T(n));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1178,10 +1218,10 @@ void lognormal_dev(mmh_ctx* c, double* rho, int n, double sigma, double slope, d
   double* sums = (double*)ws_get(c, "gen_sums", 2 * sizeof(double));
   k_white<<<nblk(n3), 256, 0, c->stream>>>(z, n3, smix_h(seed ^ 0x6A09E667F3BCC909ULL));
   LAUNCHCHK();
-  fft3_dev<double>(c, z, n, n, n, -1);
+  fft3_dev<double>(c, z, z, n, n, n, -1);
   k_pk<<<nblk(n3), 256, 0, c->stream>>>(z, n, slope, ks_frac * M_PI);
   LAUNCHCHK();
-  fft3_dev<double>(c, z, n, n, n, 1);
+  fft3_dev<double>(c, z, z, n, n, n, 1);
   k_re_sq<<<nblk(n3), 256, 0, c->stream>>>(rho, g2, z, n3);
   LAUNCHCHK();
   reduce<double>(c, g2, n3, 0, sums);
@@ -1764,9 +1804,7 @@ std::vector<double> log_edges(int n, int nb) {
 void spectrum_bins(mmh_ctx* c, const double* f, double* sd, double* sq, int n, int nb, const double* edges_dev,
                    std::vector<double>& S, std::vector<double>& N) {
   const i64 n3 = cube(n);
-  HIPCHK(hipMemcpyAsync(sd, f, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
-  fill<double>(c, sq, 0.0, 2 * (i64)n * n);
-  rlft3_dev<double>(c, sd, sq, n, 1);
+  rlft3_dev<double>(c, sd, f, sq, n, 1);
   const i64 cnt = (i64)(n / 2 + 1) * n * n;
   const unsigned nblk_ = nblk(cnt);
   double* part = (double*)ws_get(c, "pw_part", sizeof(double) * 2 * nb * (size_t)nblk_);
@@ -1888,9 +1926,7 @@ void recon_power_dev(mmh_ctx* c, const double* rho, const double* defin, int n, 
   const i64 cnt = (i64)(n / 2 + 1) * n * n;
   k_bin_filter<<<nblk(cnt), 256, 0, c->stream>>>(sd, sq, n, e, nb, symd);
   LAUNCHCHK();
-  rlft3_dev<double>(c, sd, sq, n, -1);
-  k_scale2<double><<<nblk(n3), 256, 0, c->stream>>>(w1, sd, n, n3);
-  LAUNCHCHK();
+  rlft3_dev<double>(c, sd, sd, sq, n, -1, w1, 1.0 / n);
   spectral_out<double>(c, w1, rhs, n, 1);
   if (grad_def) HIPCHK(hipMemcpyAsync(grad_def, rhs, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
   nsmooth_dev<double>(c, rhs, n, 2);
@@ -2229,7 +2265,7 @@ mmh_ctx* mmh_default_ctx(void) {
   int mmh_gradient_##S(mmh_ctx* c, const T* phi, T* psi, int n) {                                                  \
     return guarded(c, [&] {                                                                                        \
       require(is_pow2(n) && n >= 4, "gradient: n must be a power of two >= 4");                                    \
-      for (int d = 0; d < 3; ++d) spectral_out<T>(c, phi, psi + (i64)d * cube(n), n, 2 + d);                       \
+      gradient_dev<T>(c, phi, psi, n);                                                                             \
       HIPCHK(hipStreamSynchronize(c->stream));                                                                     \
     });                                                                                                            \
   }                                                                                                                \
@@ -2551,7 +2587,7 @@ int mmh_fisher_d(const double* pk, int nsim, int nk, const double* cv, double* c
 int mmh_rlft3_d(mmh_ctx* c, double* data, double* speq, int n, int isign) {
   return guarded(c, [&] {
     require(is_pow2(n) && n >= 4 && (isign == 1 || isign == -1), "rlft3: bad arguments");
-    rlft3_dev<double>(c, data, speq, n, isign);
+    rlft3_dev<double>(c, data, data, speq, n, isign);
     HIPCHK(hipStreamSynchronize(c->stream));
   });
 }
@@ -2632,7 +2668,7 @@ int mmh_gradient_host_f(mmh_ctx* c, const float* phi, float* psi, int n) {
     const i64 n3 = cube(n);
     float* a = up(c, "a", phi, n3);
     float* o = up<float>(c, "g3", nullptr, 3 * n3);
-    for (int d = 0; d < 3; ++d) spectral_out<float>(c, a, o + (i64)d * n3, n, 2 + d);
+    gradient_dev<float>(c, a, o, n);
     down(c, psi, o, 3 * n3);
     HIPCHK(hipStreamSynchronize(c->stream));
   });
