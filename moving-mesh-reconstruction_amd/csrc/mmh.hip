@@ -1090,17 +1090,20 @@ template <class T> void relaxing_dev(mmh_ctx* c, T* u, const T* def, const T* de
   require(is_pow2(n) && n >= 16 && n <= 1024, "relaxing: n must be a power of two in [16, 1024]");
   require(nf == 5, "relaxing: only nfluid = 5 is supported (relaxing.f90:307-310)");
   const i64 n3 = cube(n);
-  T* B = wsT<T>(c, "tvdB", 7 * n3);
   T* cc = wsT<T>(c, "tvdC", n3);
   T* V = wsT<T>(c, "tvdV", 15 * n3);
+  T* U = wsT<T>(c, "tvdU", 5 * n3);
   T* u1 = wsT<T>(c, "tvdU1", 5 * n3);
   const unsigned nb = nblk(n3);
-  k_binv<T><<<nb, 256, 0, c->stream>>>(B, def, n);
-  k_cfl<T><<<nb, 256, 0, c->stream>>>(cc, B, defp, u, n);
-  k_tvd_flux<T><<<nb, 256, 0, c->stream>>>(V, u, defp, B, cc, n);
-  k_tvd_step<T><<<nb, 256, 0, c->stream>>>(u1, u, u, V, cc, n, dt / T(2));
-  k_tvd_flux<T><<<nb, 256, 0, c->stream>>>(V, u1, defp, B, cc, n);
-  k_tvd_step<T><<<nb, 256, 0, c->stream>>>(u, u, u1, V, cc, n, dt);
+  // planes per workgroup of the march: the largest of 32 .. 4 that leaves 2048 workgroups (4 planes of
+  // each walk are read ahead of its first output, so short walks only where the grid is small)
+  int ks = 32;
+  while (ks > 4 && n3 / 256 / ks < 2048) ks >>= 1;
+  const unsigned nm = (unsigned)(n3 / 256 / ks);
+  k_tvd_flux<T, true><<<nb, 256, 0, c->stream>>>(V, U, cc, u, def, defp, n);
+  k_tvd_march<T, false><<<nm, 256, 0, c->stream>>>(u1, U, V, cc, n, dt / T(2), ks);
+  k_tvd_flux<T, false><<<nb, 256, 0, c->stream>>>(V, u1, cc, u, def, defp, n);
+  k_tvd_march<T, true><<<nm, 256, 0, c->stream>>>(u, u1, V, cc, n, dt, ks);
   LAUNCHCHK();
   HIPCHK(hipStreamSynchronize(c->stream));
 }
