@@ -142,7 +142,8 @@ bool batch_coarse_applies(const mmh_ctx* c, const BatchGroup& g, int l, const Sc
 
 void batch_vcycle(mmh_ctx* c, BatchGroup& g, int l, double* u0, double* rhs0, const Sched& S, const int* act = nullptr) {
   if (batch_coarse_applies(c, g, l, S)) {
-    k_coarse_stack<<<g.B, CW, 0, c->stream>>>(stack_levels(g, l, u0, rhs0, S), act);
+    if (c->coarse_lds && g.m[l] <= 16) k_coarse16_stack<<<g.B, CW, 0, c->stream>>>(stack_levels(g, l, u0, rhs0, S), act);
+    else k_coarse_stack<<<g.B, CW, 0, c->stream>>>(stack_levels(g, l, u0, rhs0, S), act);
     LAUNCHCHK();
     return;
   }

@@ -18,7 +18,7 @@
 
 namespace mmh {
 
-constexpr int CW = 512;        // threads of the coarse-cycle workgroup (1024 and 256 measured slower)
+constexpr int CW = 512;        // threads of the coarse-cycle workgroup (1024 and 256 measured slower for this form)
 constexpr int CLEV_MAX = 8;    // levels one coarse cycle may hold
 constexpr int CTOP_MAX = 32;   // largest level run this way (its sums have <= 16 blocks)
 

@@ -30,6 +30,7 @@
 #include "kernels_vis.hpp"
 #include "kernels_march.hpp"
 #include "kernels_coarse.hpp"
+#include "kernels_coarse16.hpp"
 #include "kernels_gal.hpp"
 
 #include <hipcub/hipcub.hpp>
@@ -685,6 +686,20 @@ template <class T> CoarseCycle<T> coarse_cycle_of(Hier<T>& H, int l, const Sched
   return C;
 }
 
+// The cycle's launch: levels from 16^3 down are laid out on chip (k_coarse16); with a 32^3 level (option
+// "coarse_fused" or "coarse_fused_ref" 32), or option "coarse_lds" 0, the general one-workgroup form runs.
+template <class T> void coarse_cycle_launch(mmh_ctx* c, CoarseCycle<T>& C) {
+  if (!c->coarse_lds) {
+    k_coarse_cycle<T><<<1, CW, 0, c->stream>>>(C);
+  } else if (C.n[0] <= 16) {
+    k_coarse16<T><<<1, CW, 0, c->stream>>>(C);
+  } else {
+    stage_levels(C);
+    k_coarse_cycle_lds<T><<<1, CW, 0, c->stream>>>(C);
+  }
+  LAUNCHCHK();
+}
+
 // One V-cycle from level l (mgtemplate.f90 / mg*.f90; mg4 at multigrid.f90:94-121).
 template <class T> void vcycle(mmh_ctx* c, Hier<T>& H, int l, int ng_top, const Sched& S) {
   const int n = H.n[l];
@@ -692,13 +707,7 @@ template <class T> void vcycle(mmh_ctx* c, Hier<T>& H, int l, int ng_top, const 
   double* sc = H.scal + 3 * l;
   if (coarse_cycle_applies(c, H, l, S)) {
     CoarseCycle<T> C = coarse_cycle_of(H, l, S, ng_top);
-    if (c->coarse_lds) {
-      stage_levels(C);
-      k_coarse_cycle_lds<T><<<1, CW, 0, c->stream>>>(C);
-    } else {
-      k_coarse_cycle<T><<<1, CW, 0, c->stream>>>(C);
-    }
-    LAUNCHCHK();
+    coarse_cycle_launch<T>(c, C);
     return;
   }
   const bool zero = c->zero_start && (l > 0 || S.top_zero);
@@ -1279,13 +1288,7 @@ void vcycle_mixed(mmh_ctx* c, Hier<float>& Hf, Hier<double>& Hd, int l, int ng_t
     C.dguard = Hd.guard + lb;
     C.ddx = Hd.dx[lb];
     C.dA = Hd.A[lb];
-    if (c->coarse_lds) {
-      stage_levels(C);
-      k_coarse_cycle_lds<float><<<1, CW, 0, c->stream>>>(C);
-    } else {
-      k_coarse_cycle<float><<<1, CW, 0, c->stream>>>(C);
-    }
-    LAUNCHCHK();
+    coarse_cycle_launch<float>(c, C);
     return;
   }
   if (n == 4) {
