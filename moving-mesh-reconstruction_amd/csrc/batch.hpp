@@ -71,19 +71,16 @@ void batch_sweeps(mmh_ctx* c, BatchGroup& g, double* phi, const double* rhs, con
   const i64 h3 = cube(m / 2);
   const double dx2 = g.dx[l] * g.dx[l];
   const int bsz = shape.first;
-  const dim3 grid(nblk(h3, bsz), g.B);
-  for (int sw = 0; sw < ns; ++sw)
-    for (int cc = 0, done = 0; cc < 8; ++cc) {
-      const int col = reverse ? 7 - cc : cc;
-      if (sw == 0 && from_zero)
-        k_colour<double, 1, false, true><<<grid, bsz, 0, c->stream>>>(phi, rhs, G, m, dx2, col >> 2, (col >> 1) & 1,
-                                                                      col & 1, cube(m), shape.second, (unsigned)done,
-                                                                      act);
-      else
-        k_colour<double, 1><<<grid, bsz, 0, c->stream>>>(phi, rhs, G, m, dx2, col >> 2, (col >> 1) & 1, col & 1, cube(m),
-                                                         shape.second, 0xFFu, act);
-      done |= 1 << col;
-    }
+  const unsigned nb = nblk(h3, bsz);
+  colour_steps(ns, reverse, true, from_zero, [&](int col, bool pair, bool first, unsigned done) {
+    const dim3 grid(pair ? 2 * nb : nb, g.B);
+    if (first && from_zero)
+      k_colour<double, 1, false, true><<<grid, bsz, 0, c->stream>>>(phi, rhs, G, m, dx2, col >> 2, (col >> 1) & 1, col & 1,
+                                                                    cube(m), shape.second, done, act, pair);
+    else
+      k_colour<double, 1><<<grid, bsz, 0, c->stream>>>(phi, rhs, G, m, dx2, col >> 2, (col >> 1) & 1, col & 1, cube(m),
+                                                       shape.second, 0xFFu, act, pair);
+  });
   LAUNCHCHK();
 }
 

@@ -416,16 +416,28 @@ __device__ __forceinline__ void colour_point(T* __restrict__ phi, const T* __res
 // Batched launches: gridDim.y = B grids of the same size stored one after another (bstride = n^3
 // values; G holds 6 n^3 per grid).  remap = 0 keeps the hardware's block order (a tuning choice).
 // MASK: the first sweep from phi = 0, where live holds the classes updated earlier in the sweep.
+// pair: the second half of the blocks updates the complementary class (all three parities flipped), which
+// the 19-point operator does not couple to the first: two colours in one launch where they follow
+// each other (colour_steps), the same values.
 template <class T, int L, bool DELTA = false, bool MASK = false, class TG = T>
 __global__ __launch_bounds__(256) void k_colour(T* __restrict__ phi, const T* __restrict__ rhs, const TG* __restrict__ G, int n,
                                                 T dx2, int kpar, int io, int jo, i64 bstride = 0, int remap = 1,
-                                                unsigned live = 0xFFu, const int* __restrict__ act = nullptr) {
+                                                unsigned live = 0xFFu, const int* __restrict__ act = nullptr,
+                                                int pair = 0) {
   if (act && !act[blockIdx.y]) return;  // a grid of a batch that has converged
   const int h = n >> 1;
+  unsigned bx = blockIdx.x, nbx = gridDim.x;
+  if (pair) {
+    nbx >>= 1;
+    if (bx >= nbx) {
+      bx -= nbx;
+      kpar ^= 1; io ^= 1; jo ^= 1;
+    }
+  }
   phi += (i64)blockIdx.y * bstride;
   rhs += (i64)blockIdx.y * bstride;
   G += (i64)blockIdx.y * 6 * bstride;
-  const unsigned blk = remap ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+  const unsigned blk = remap ? xcd_remap(bx, nbx) : bx;
   const i64 q = (i64)blk * blockDim.x + threadIdx.x;
   if (q >= (i64)h * h * h) return;
   colour_point<T, L, DELTA, MASK, TG>(phi, rhs, G, n, dx2, kpar, io, jo, q, live);
