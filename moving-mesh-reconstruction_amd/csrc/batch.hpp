@@ -380,8 +380,8 @@ void batch_setup_group(mmh_ctx* c, BatchGroup& g, std::vector<const void*>& tab,
   batch_reduce(c, g, rst, n3, 1, rnmax);
   k_scatter<double><<<gr, 256, 0, c->stream>>>(t_rhs, rst, n3);
   k_gather<double><<<gr, 256, 0, c->stream>>>(det, t_u, n3, 1);  // det is free again
-  k_relayout<double, 1><<<gr, 256, 0, c->stream>>>(g.x, det, n, 1, 1);
-  k_relayout<double, 1><<<gr, 256, 0, c->stream>>>(g.b, rst, n, 1, 1);
+  k_relayout<double, 1><<<dim3(nblk(n3 / 2), B), 256, 0, c->stream>>>(g.x, det, n, 1);
+  k_relayout<double, 1><<<dim3(nblk(n3 / 2), B), 256, 0, c->stream>>>(g.b, rst, n, 1);
   LAUNCHCHK();
 }
 

@@ -186,23 +186,31 @@ template <int L, bool SM = false> __device__ __forceinline__ void point_of(i64 p
   k = 2 * (int)(q / ((i64)h * h)) + ((c >> 2) & 1);
 }
 
+// TO = 1: column-major -> sub-lattice; TO = 0: sub-lattice -> column-major; a field of n^3 (batched: grid y
+// of gridDim.y at y n^3).  A thread moves the two points of an x pair, adjacent in the one layout and
+// unit-stride in two class arrays of the other, so both sides use whole lines (a thread per point
+// read every line of the column-major side twice): 512^3 FP32 547 -> 182 us.
 template <class T, int TO>
-__global__ void k_relayout(T* __restrict__ dst, const T* __restrict__ src, int n, int comps, int batched = 0) {
-  // TO = 1: column-major -> sub-lattice; TO = 0: sub-lattice -> column-major; comps fields of n^3
-  // (batched: grid y of gridDim.y at y comps n^3)
-  const i64 n3 = (i64)n * n * n;
+__global__ __launch_bounds__(256) void k_relayout(T* __restrict__ dst, const T* __restrict__ src, int n, int batched = 0) {
+  const int lg = __builtin_ctz(n), h = n >> 1;
+  const i64 n3 = (i64)1 << (3 * lg), h3 = n3 >> 3;
   if (batched) {
-    dst += (i64)blockIdx.y * comps * n3;
-    src += (i64)blockIdx.y * comps * n3;
+    dst += (i64)blockIdx.y * n3;
+    src += (i64)blockIdx.y * n3;
   }
-  const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n3 * comps) return;
-  const int f = (int)(p / n3);
-  int i, j, k;
-  point_of<1>(p - f * n3, n, i, j, k);
-  const i64 a = f * n3 + lx<1>(i, j, k, n), b = f * n3 + ix3(i, j, k, n);
-  if (TO == 1) dst[a] = src[b];
-  else dst[b] = src[a];
+  const i64 q = (i64)blockIdx.x * blockDim.x + threadIdx.x;  // pair, x fastest
+  if (q >= (n3 >> 1)) return;
+  const int x = (int)(q & (h - 1)), j = (int)(q >> (lg - 1)) & (n - 1), k = (int)(q >> (2 * lg - 1));
+  const i64 a = ((i64)((j & 1) << 1 | (k & 1) << 2)) * h3 + x + (i64)h * ((j >> 1) + (i64)h * (k >> 1)), b = 2 * q;
+  if (TO == 1) {
+    const T v0 = src[b], v1 = src[b + 1];
+    dst[a] = v0;
+    dst[a + h3] = v1;
+  } else {
+    const T v0 = src[a], v1 = src[a + h3];
+    dst[b] = v0;
+    dst[b + 1] = v1;
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1053,12 +1061,40 @@ __global__ __launch_bounds__(256) void k_restrict27(T* __restrict__ half, const 
   half[q] = box27(full, stride, n, 2 * i, 2 * j, 2 * k);
 }
 
-template <class T>
+// nsmooth (mmh/limiter.f90:677) out of place: a thread walks KS planes of one (i, j) column with the nine
+// values of three planes in registers, so a point loads nine values instead of 27 and the pass is
+// bound by memory.  512^3 FP32: 780 -> 379 us (368 with KS = 16).  n a power of two, KS divides n.
+template <class T, int KS>
 __global__ __launch_bounds__(256) void k_smooth27(T* __restrict__ out, const T* __restrict__ in, int n) {
-  const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= (i64)n * n * n) return;
-  const int i = (int)(p % n), j = (int)((p / n) % n), k = (int)(p / ((i64)n * n));
-  out[p] = box27(in, 1, n, i, j, k);
+  const int lg = __builtin_ctz(n), m = n - 1;
+  const unsigned gx = (unsigned)(n * n + 255) >> 8, blk = xcd_remap(blockIdx.x, gridDim.x);
+  const int seg = (int)(blk / gx), r = (int)(blk - (unsigned)seg * gx) * 256 + (int)threadIdx.x;
+  if (r >= n * n) return;
+  const int i = r & m, j = r >> lg;
+  const int xs[3] = {(i - 1) & m, i, (i + 1) & m}, ys[3] = {((j - 1) & m) << lg, j << lg, ((j + 1) & m) << lg};
+  uint32_t o[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) o[q] = (uint32_t)(xs[q % 3] + ys[q / 3]) * (uint32_t)sizeof(T);
+  T v[3][9];  // planes k - 1, k, k + 1 at [(k + 2) % 3] ..
+  auto load = [&](T (&w)[9], int k) {
+    const char* base = (const char*)(in + ((i64)(k & m) << (2 * lg)));
+#pragma unroll
+    for (int q = 0; q < 9; ++q) w[q] = *(const T*)(base + o[q]);
+  };
+  const int k0 = seg * KS;
+  load(v[0], k0 - 1);
+  load(v[1], k0);
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    load(v[(s + 2) % 3], k0 + s + 1);
+    const T (&M)[9] = v[s % 3], (&C)[9] = v[(s + 1) % 3], (&P)[9] = v[(s + 2) % 3];
+    // box27's terms: index 4 the point, 5 / 3 its i + 1 / i - 1, 7 / 1 its j + 1 / j - 1
+    const T t = C[4] / T(8)
+      + (C[5] + C[3] + C[7] + C[1] + P[4] + M[4]) / T(16)
+      + (C[8] + C[2] + C[6] + C[0] + P[5] + M[5] + P[3] + M[3] + P[7] + M[7] + P[1] + M[1]) / T(32)
+      + (P[8] + M[8] + P[2] + M[2] + P[6] + M[6] + P[0] + M[0]) / T(64);
+    *(T*)((char*)(out + ((i64)(k0 + s) << (2 * lg))) + o[4]) = t;
+  }
 }
 
 // Trilinear prolongation (mmh/mgutil.f90:38-71 inject adds; 2-34 prolong overwrites); u (n^3) and
@@ -1152,8 +1188,9 @@ __global__ __launch_bounds__(256) void k_det(T* __restrict__ det, const T* __res
   }
   const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= (i64)n * n * n) return;
-  const int i = (int)(p % n), j = (int)((p / n) % n), k = (int)(p / ((i64)n * n));
-  const int ip = wrapi(i + 1, n), im = wrapi(i - 1, n), jp = wrapi(j + 1, n), jm = wrapi(j - 1, n), kp = wrapi(k + 1, n), km = wrapi(k - 1, n);
+  const int lg = __builtin_ctz(n), m = n - 1;  // n a power of two
+  const int i = (int)p & m, j = (int)(p >> lg) & m, k = (int)(p >> (2 * lg));
+  const int ip = (i + 1) & m, im = (i - 1) & m, jp = (j + 1) & m, jm = (j - 1) & m, kp = (k + 1) & m, km = (k - 1) & m;
   const T di2 = T(1) / (dx * dx);
   const T d0 = def[p];
   T phixx = (def[ix3(ip, j, k, n)] - T(2) * d0 + def[ix3(im, j, k, n)]) * di2;

@@ -148,7 +148,7 @@ __global__ void k_adj_metric(double* __restrict__ grhobar, double* __restrict__ 
   const double wxy = -0.25 * (dly * dfx + dlx * dfy);
   const double wxz = -0.25 * (dlz * dfx + dlx * dfz);
   const double wyz = -0.25 * (dlz * dfy + dly * dfz);
-  const Hs<double> h = hess(def, n, i, j, k);
+  const Hs<double> h = hess(def, PlanePoint(n, blockIdx.x));
   const double a11 = 1.0 + h.xx, a12 = h.xy, a13 = h.xz, a22 = 1.0 + h.yy, a23 = h.yz, a33 = 1.0 + h.zz;
   const double det = a11 * a22 * a33 + 2.0 * a12 * a13 * a23 - a13 * a13 * a22 - a11 * a23 * a23 - a12 * a12 * a33;
   // adj(A) (cofactors, symmetric)

@@ -8,38 +8,41 @@ namespace mmh {
 
 template <class T> struct Hs { T xx, yy, zz, xy, yz, xz; };
 
+// Point threadIdx.x of the 256-point chunk `chunk` of a field whose n is a power of two and n^2 a multiple of
+// 256: the chunk lies in one plane, so plane bases are scalars and a lane adds its 32-bit offset.
+struct PlanePoint {
+  int lg, m, k;
+  i64 pl;      // first point of the plane
+  unsigned r;  // index in the plane
+  int xs[3], ys[3];
+  __device__ __forceinline__ PlanePoint(int n, i64 chunk) : lg(__builtin_ctz(n)), m(n - 1) {
+    const i64 p0 = chunk * 256;
+    k = (int)(p0 >> (2 * lg));
+    pl = (i64)k << (2 * lg);
+    r = (unsigned)(p0 - pl) + threadIdx.x;
+    const int i = (int)r & m, j = (int)(r >> lg);
+    xs[0] = (i - 1) & m; xs[1] = i; xs[2] = (i + 1) & m;
+    ys[0] = ((j - 1) & m) << lg; ys[1] = j << lg; ys[2] = ((j + 1) & m) << lg;
+  }
+  template <class T> __device__ __forceinline__ T at(const T* f, int di, int dj, int dk) const {
+    return *(const T*)((const char*)(f + ((i64)((k + dk) & m) << (2 * lg))) +
+                       (uint32_t)(xs[di + 1] + ys[dj + 1]) * (uint32_t)sizeof(T));
+  }
+  template <class T> __device__ __forceinline__ void put(T* f, T v) const {
+    *(T*)((char*)(f + pl) + r * (uint32_t)sizeof(T)) = v;
+  }
+};
 // Hessian stencil without grid scaling (mmh/limiter.f90:268-273, mmh/relaxing.f90:876-881).
-template <class T> __device__ __forceinline__ Hs<T> hess(const T* __restrict__ f, int n, int i, int j, int k) {
-  const int ip = wrapi(i + 1, n), im = wrapi(i - 1, n), jp = wrapi(j + 1, n), jm = wrapi(j - 1, n), kp = wrapi(k + 1, n), km = wrapi(k - 1, n);
-  const T f0 = f[ix3(i, j, k, n)];
+template <class T> __device__ __forceinline__ Hs<T> hess(const T* __restrict__ f, const PlanePoint& P) {
+  const T f0 = P.at(f, 0, 0, 0);
   Hs<T> h;
-  h.xx = (f[ix3(ip, j, k, n)] - T(2) * f0 + f[ix3(im, j, k, n)]);
-  h.yy = (f[ix3(i, jp, k, n)] - T(2) * f0 + f[ix3(i, jm, k, n)]);
-  h.zz = (f[ix3(i, j, kp, n)] - T(2) * f0 + f[ix3(i, j, km, n)]);
-  h.xy = (f[ix3(ip, jp, k, n)] - f[ix3(im, jp, k, n)] - f[ix3(ip, jm, k, n)] + f[ix3(im, jm, k, n)]) / T(4);
-  h.yz = (f[ix3(i, jp, kp, n)] - f[ix3(i, jp, km, n)] - f[ix3(i, jm, kp, n)] + f[ix3(i, jm, km, n)]) / T(4);
-  h.xz = (f[ix3(ip, j, kp, n)] - f[ix3(im, j, kp, n)] - f[ix3(ip, j, km, n)] + f[ix3(im, j, km, n)]) / T(4);
+  h.xx = (P.at(f, 1, 0, 0) - T(2) * f0 + P.at(f, -1, 0, 0));
+  h.yy = (P.at(f, 0, 1, 0) - T(2) * f0 + P.at(f, 0, -1, 0));
+  h.zz = (P.at(f, 0, 0, 1) - T(2) * f0 + P.at(f, 0, 0, -1));
+  h.xy = (P.at(f, 1, 1, 0) - P.at(f, -1, 1, 0) - P.at(f, 1, -1, 0) + P.at(f, -1, -1, 0)) / T(4);
+  h.yz = (P.at(f, 0, 1, 1) - P.at(f, 0, 1, -1) - P.at(f, 0, -1, 1) + P.at(f, 0, -1, -1)) / T(4);
+  h.xz = (P.at(f, 1, 0, 1) - P.at(f, -1, 0, 1) - P.at(f, 1, 0, -1) + P.at(f, -1, 0, -1)) / T(4);
   return h;
-}
-
-// b = adj(A)/det, det, A = I + H, no clamp (mmh/limiter.f90:274-286, mmh/relaxing.f90:882-901).
-// B planes: 0..5 = b11,b12,b13,b22,b23,b33, 6 = det.
-template <class T>
-__global__ __launch_bounds__(256) void k_binv(T* __restrict__ B, const T* __restrict__ def, int n) {
-  const i64 n3 = (i64)n * n * n;
-  const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n3) return;
-  const int i = (int)(p % n), j = (int)((p / n) % n), k = (int)(p / ((i64)n * n));
-  Hs<T> h = hess(def, n, i, j, k);
-  T a11 = T(1) + h.xx, a12 = h.xy, a13 = h.xz, a22 = T(1) + h.yy, a23 = h.yz, a33 = T(1) + h.zz;
-  T det = a11 * a22 * a33 + T(2) * a12 * a13 * a23 - (a13 * a13) * a22 - a11 * (a23 * a23) - (a12 * a12) * a33;
-  B[0 * n3 + p] = (a22 * a33 - a23 * a23) / det;
-  B[1 * n3 + p] = (a13 * a23 - a12 * a33) / det;
-  B[2 * n3 + p] = (a12 * a23 - a13 * a22) / det;
-  B[3 * n3 + p] = (a11 * a33 - a13 * a13) / det;
-  B[4 * n3 + p] = (a12 * a13 - a11 * a23) / det;
-  B[5 * n3 + p] = (a11 * a22 - a12 * a12) / det;
-  B[6 * n3 + p] = det;
 }
 
 // Smallest eigenvalue of symmetric C by the trigonometric method; returns 1/lambda_min
@@ -57,119 +60,165 @@ __device__ __forceinline__ T compression_of(T c11, T c12, T c13, T c22, T c23, T
   T arg = T(3) * b / a / am;
   arg = dmax(T(-1.), dmin(T(1.), arg));
   T theta = acos(arg) / T(3);
-  T r1 = am * cos(theta);
-  T r2 = am * cos(theta + T(2) * pi / T(3.));
-  T r3 = am * cos(theta + T(4) * pi / T(3.));
+  // The three roots are am cos(theta + 0, 2 pi/3, 4 pi/3) with theta in [0, pi/3]: the first is the largest,
+  // and the third exceeds the second by sqrt(3) am sin(theta), far above rounding unless theta is
+  // small, so only there is the third formed (and the smaller taken); the value is that of the
+  // minimum over all three.
   T t3 = trace / T(3);
-  T l1 = r1 + t3, l2 = r2 + t3, l3 = r3 + t3;
-  return T(1) / dmin(dmin(l1, l2), l3);
+  T l2 = am * cos(theta + T(2) * pi / T(3.)) + t3;
+  if (!(theta > T(0.01))) {
+    T l3 = am * cos(theta + T(4) * pi / T(3.)) + t3;
+    l2 = dmin(l2, l3);
+  }
+  return T(1) / l2;
 }
 
-// Step 1 of calcdefp: clipped, scaled mass mismatch (mmh/limiter.f90:134-169).
+// Step 1 of calcdefp: clipped, scaled mass mismatch (mmh/limiter.f90:134-169).  rho (may be null): the
+// density itself, contiguous, for the metric's box mean (u is read once for both).
 template <class T>
-__global__ void k_mismatch(T* __restrict__ tmp, const T* __restrict__ u, int nf, i64 n3, T dtold) {
+__global__ void k_mismatch(T* __restrict__ tmp, T* __restrict__ rho, const T* __restrict__ u, int nf, i64 n3, T dtold) {
   const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n3) return;
   const T u1 = u[(i64)nf * p];
+  if (rho) rho[p] = u1;
   T t1 = T(1.0f) - u1;
   const T xhigh = 2;
   if (fabs(t1) > xhigh) t1 = copysign(xhigh, t1);
   tmp[p] = t1 / T(30) / dtold;
 }
 
-// Step 3 of calcdefp: the eflux of plane k-1 from the metric and eigenvalues of plane k
-// (mmh/limiter.f90:238-381), including the expansion limiter (det > 10) and the compression gate.
-// stat: per-block [nexpand, detmax, detmin, fluxmax, fluxmin] combined by the host.
+// Diagnostics of a workgroup: thread values combined over the wavefront and then the workgroup, stored
+// at part[f gridDim.x + block].  Maxima, minima and counts do not depend on the order.
+template <int OP> __device__ __forceinline__ double stat_op(double a, double b) {
+  return OP == 0 ? a + b : (OP == 1 ? dmax(a, b) : dmin(a, b));
+}
+template <int OP> __device__ __forceinline__ void block_stat(double a, double* part, int f) {
+  __shared__ double w[4];
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) a = stat_op<OP>(a, __shfl_xor(a, h));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    part[(i64)f * gridDim.x + blockIdx.x] = stat_op<OP>(stat_op<OP>(w[0], w[1]), stat_op<OP>(w[2], w[3]));
+}
+// The same over nb block results per field, in field order, by gridDim.x workgroups of 256.
+__global__ __launch_bounds__(256) void k_stats(double* __restrict__ out, const double* __restrict__ part, i64 nb, int nf,
+                                               unsigned ops) {
+  for (int f = 0; f < nf; ++f) {
+    const unsigned op = (ops >> (2 * f)) & 3u;
+    i64 b = (i64)blockIdx.x * 256 + threadIdx.x;
+    double a = op == 0 ? 0.0 : part[f * nb + (b < nb ? b : 0)];  // a repeated value changes no maximum or minimum
+    if (op == 0 && b < nb) a = part[f * nb + b];
+    for (b += (i64)gridDim.x * 256; b < nb; b += (i64)gridDim.x * 256) {
+      const double v = part[f * nb + b];
+      a = op == 0 ? a + v : (op == 1 ? dmax(a, v) : dmin(a, v));
+    }
+    if (op == 0) block_stat<0>(a, out, f);
+    else if (op == 1) block_stat<1>(a, out, f);
+    else block_stat<2>(a, out, f);
+  }
+}
+
+// Points of a thread of the limiter's kernels (n >= 16, so n^3 is a multiple of 256 LIM_PT): 256 LIM_PT
+// consecutive points per workgroup, so that the
+// block results stay few (at one point per thread the host read and combined 20 MB of them at 512^3).
+constexpr int LIM_PT = 4;
+
+// Step 3 of calcdefp (mmh/limiter.f90:238-381), pointwise part: the three components of the fluid's flux,
+// s_d = (b_d . momentum) / rho with b = adj(A)/det, A = I + H(def) (limiter.f90:274-286), and which of
+// the expansion limiter (det > 10, flag bit 0) and the compression gate (bit 1) hold at the point.
+// The metric is formed and used in one pass; forming it at the flux's six neighbours from a stored
+// metric took 5.1 ms with that pass at 512^3 FP32, the two passes now 1.43 + 0.50 ms.
+// part: per workgroup nexpand, detmax, detmin.  n a power of two, n^2 a multiple of 256.
 template <class T>
-__global__ __launch_bounds__(256) void k_eflux(T* __restrict__ eflux, const T* __restrict__ tmp, const T* __restrict__ B,
-                                               const T* __restrict__ def, const T* __restrict__ u, int nf, int n, T dtold,
-                                               T dtaumesh, T cmpmaxglobal, T pi, double* __restrict__ bstat,
-                                               T* __restrict__ gate = nullptr) {
-  __shared__ double s[5][256];
+__global__ __launch_bounds__(256) void k_lim_point(T* __restrict__ s, unsigned char* __restrict__ flag,
+                                                   const T* __restrict__ def, const T* __restrict__ u, int nf, int n, T dtold,
+                                                   T cmpmaxglobal, T pi, double* __restrict__ part) {
   const i64 n3 = (i64)n * n * n;
-  const i64 pk = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-  double st[5] = {0.0, 0.0, 1.0, 0.0, 0.0};
-  if (pk < n3) {
-    const int i = (int)(pk % n), j = (int)((pk / n) % n), k = (int)(pk / ((i64)n * n));
-    const int km = wrapi(k - 1, n), kmm = wrapi(k - 2, n);
-    const int ip = wrapi(i + 1, n), im = wrapi(i - 1, n), jp = wrapi(j + 1, n), jm = wrapi(j - 1, n);
-    const i64 pkm = ix3(i, j, km, n);
-    const T det = B[6 * n3 + pk];
-    const T b13 = B[2 * n3 + pk], b23 = B[4 * n3 + pk], b33 = B[5 * n3 + pk];
-#define BM(c, a, b2, kk) B[(i64)(c) * n3 + ix3(a, b2, kk, n)]
-#define UU(c, pp) u[(i64)nf * (pp) + (c)]
-    i64 q;
-    q = ix3(ip, j, km, n);
-    T s1p = (BM(0, ip, j, km) * UU(1, q) + BM(1, ip, j, km) * UU(2, q) + BM(2, ip, j, km) * UU(3, q)) / UU(0, q);
-    q = ix3(i, jp, km, n);
-    T s2p = (BM(1, i, jp, km) * UU(1, q) + BM(3, i, jp, km) * UU(2, q) + BM(4, i, jp, km) * UU(3, q)) / UU(0, q);
-    T s3p = (b13 * UU(1, pk) + b23 * UU(2, pk) + b33 * UU(3, pk)) / UU(0, pk);
-    q = ix3(im, j, km, n);
-    T s1m = (BM(0, im, j, km) * UU(1, q) + BM(1, im, j, km) * UU(2, q) + BM(2, im, j, km) * UU(3, q)) / UU(0, q);
-    q = ix3(i, jm, km, n);
-    T s2m = (BM(1, i, jm, km) * UU(1, q) + BM(3, i, jm, km) * UU(2, q) + BM(4, i, jm, km) * UU(3, q)) / UU(0, q);
-    q = ix3(i, j, kmm, n);
-    T s3m = (BM(2, i, j, kmm) * UU(1, q) + BM(4, i, j, kmm) * UU(2, q) + BM(5, i, j, kmm) * UU(3, q)) / UU(0, q);
-#undef BM
-#undef UU
+  double nexp = 0.0, dhi = 0.0, dlo = 1.0;
+  const i64 chunk0 = (i64)xcd_remap(blockIdx.x, gridDim.x) * LIM_PT;
+  for (int q = 0; q < LIM_PT; ++q) {
+    const PlanePoint P(n, chunk0 + q);
+    const Hs<T> h = hess(def, P);
+    const T a11 = T(1) + h.xx, a12 = h.xy, a13 = h.xz, a22 = T(1) + h.yy, a23 = h.yz, a33 = T(1) + h.zz;
+    const T det = a11 * a22 * a33 + T(2) * a12 * a13 * a23 - (a13 * a13) * a22 - a11 * (a23 * a23) - (a12 * a12) * a33;
+    const T b11 = (a22 * a33 - a23 * a23) / det;
+    const T b12 = (a13 * a23 - a12 * a33) / det;
+    const T b13 = (a12 * a23 - a13 * a22) / det;
+    const T b22 = (a11 * a33 - a13 * a13) / det;
+    const T b23 = (a12 * a13 - a11 * a23) / det;
+    const T b33 = (a11 * a22 - a12 * a12) / det;
+    const T* ul = u + (i64)nf * (P.pl + P.r);
+    const T u0 = ul[0], u1 = ul[1], u2 = ul[2], u3 = ul[3];
+    P.put(s, (b11 * u1 + b12 * u2 + b13 * u3) / u0);
+    P.put(s + n3, (b12 * u1 + b22 * u2 + b23 * u3) / u0);
+    P.put(s + 2 * n3, (b13 * u1 + b23 * u2 + b33 * u3) / u0);
+    const T compression = compression_of(a11, a12, a13, a22, a23, a33, pi);
+    const T cmpmax = cmpmaxglobal * T(1);
+    const T tlim = T(3) * (T(1) / cmpmax - T(1) / compression) / dtold;
+    const bool ex = det > T(10.0f);
+    P.put(flag, (unsigned char)((ex ? 1 : 0) | (tlim > T(0) ? 2 : 0)));
+    nexp += ex ? 1.0 : 0.0;
+    dhi = dmax(dhi, (double)det);
+    dlo = dmin(dlo, (double)det);
+  }
+  block_stat<0>(nexp, part, 0);
+  block_stat<1>(dhi, part, 1);
+  block_stat<2>(dlo, part, 2);
+}
+
+// The eflux of a point from the fluxes of its neighbours and the gates of the point one plane above
+// it (limiter.f90:330-381); gate: the derivative of this eflux with respect to the smoothed mismatch
+// tmp at fixed def (the expansion limiter's -2|.|, the compression gate's max(0, .) and the clamp, each
+// taken on the branch the forward pass took; the e.v terms vanish with u(2:4) = 0).
+// part: per workgroup fluxmax, fluxmin.
+template <class T>
+__global__ __launch_bounds__(256) void k_eflux(T* __restrict__ eflux, const T* __restrict__ tmp, const T* __restrict__ s,
+                                               const unsigned char* __restrict__ flag, int n, T dtold, T dtaumesh,
+                                               double* __restrict__ part, T* __restrict__ gate) {
+  const i64 n3 = (i64)n * n * n;
+  double fhi = 0.0, flo = 0.0;
+  const i64 chunk0 = (i64)xcd_remap(blockIdx.x, gridDim.x) * LIM_PT;
+  for (int q = 0; q < LIM_PT; ++q) {
+    const PlanePoint P(n, chunk0 + q);
+    const T s1p = P.at(s, 1, 0, 0), s1m = P.at(s, -1, 0, 0);
+    const T s2p = P.at(s + n3, 0, 1, 0), s2m = P.at(s + n3, 0, -1, 0);
+    const T s3p = P.at(s + 2 * n3, 0, 0, 1), s3m = P.at(s + 2 * n3, 0, 0, -1);
     T ef = (s1p + s2p + s3p - s1m - s2m - s3m) / T(2);
-    ef = ef + tmp[pkm];
-    // d eflux / d tmp with every gate frozen at its branch (the adjoint's use; see gate below)
+    ef = ef + P.at(tmp, 0, 0, 0);
+    const unsigned g = P.at(flag, 0, 0, 1);
     T dm = T(1);
-    if (det > T(10.0f)) {
+    if (g & 1u) {
       dm = ef > T(0) ? -T(2) : (ef < T(0) ? T(2) : T(0));
       ef = -T(2) * fabs(ef);
-      st[0] = 1.0;
     }
-    Hs<T> h = hess(def, n, i, j, k);
-    T compression = compression_of(T(1) + h.xx, h.xy, h.xz, T(1) + h.yy, h.yz, T(1) + h.zz, pi);
-    T cmpmax = cmpmaxglobal * T(1);
-    T tlim = T(3) * (T(1) / cmpmax - T(1) / compression) / dtold;
-    if (tlim > T(0)) {
+    if (g & 2u) {
       if (!(ef > T(0))) dm = T(0);
       ef = dmax(T(0.), ef);
     }
-    st[1] = (double)det;
-    st[2] = (double)det;
     if (!(ef < T(1.) / dtaumesh && ef > -T(1.) / dtaumesh)) dm = T(0);
     ef = dmin(T(1.) / dtaumesh, ef);
     ef = dmax(-T(1.) / dtaumesh, ef);
-    eflux[pkm] = ef;
-    // gate: the derivative of this eflux with respect to the smoothed mismatch tmp[pkm] at fixed
-    // def (the expansion limiter's -2|.|, the compression gate's max(0, .) and the clamp, each
-    // taken on the branch the forward pass took; the e.v terms vanish with u(2:4) = 0)
-    if (gate) gate[pkm] = dm;
-    st[3] = (double)(ef * dtold);
-    st[4] = (double)(ef * dtold);
+    P.put(eflux, ef);
+    if (gate) P.put(gate, dm);
+    fhi = dmax(fhi, (double)(ef * dtold));
+    flo = dmin(flo, (double)(ef * dtold));
   }
-  for (int c = 0; c < 5; ++c) s[c][threadIdx.x] = st[c];
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      s[0][threadIdx.x] += s[0][threadIdx.x + h];
-      s[1][threadIdx.x] = dmax(s[1][threadIdx.x], s[1][threadIdx.x + h]);
-      s[2][threadIdx.x] = dmin(s[2][threadIdx.x], s[2][threadIdx.x + h]);
-      s[3][threadIdx.x] = dmax(s[3][threadIdx.x], s[3][threadIdx.x + h]);
-      s[4][threadIdx.x] = dmin(s[4][threadIdx.x], s[4][threadIdx.x + h]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    for (int c = 0; c < 5; ++c) bstat[5 * (i64)blockIdx.x + c] = s[c][0];
+  block_stat<1>(fhi, part, 0);
+  block_stat<2>(flo, part, 1);
 }
 
 // Step 5 of calcdefp: compression limiter source (mmh/limiter.f90:425-533).  lim = tlim where
-// lambda_min(I + H(def) + dtold*H(defp)) < 1/cmpmax; per-block [ncompress, cmax].
+// lambda_min(I + H(def) + dtold*H(defp)) < 1/cmpmax; part: per workgroup ncompress, cmax.
 template <class T>
 __global__ __launch_bounds__(256) void k_complim(T* __restrict__ lim, const T* __restrict__ defp, const T* __restrict__ def,
-                                                 int n, T dtold, T cmpmaxglobal, T pi, double* __restrict__ bstat) {
-  __shared__ double s[2][256];
-  const i64 n3 = (i64)n * n * n;
-  const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+                                                 int n, T dtold, T cmpmaxglobal, T pi, double* __restrict__ part) {
   double c0 = 0.0, c1 = 0.0;
-  if (p < n3) {
-    const int i = (int)(p % n), j = (int)((p / n) % n), k = (int)(p / ((i64)n * n));
-    Hs<T> hp = hess(defp, n, i, j, k), hd = hess(def, n, i, j, k);
+  const i64 chunk0 = (i64)xcd_remap(blockIdx.x, gridDim.x) * LIM_PT;
+  for (int q = 0; q < LIM_PT; ++q) {
+    const PlanePoint P(n, chunk0 + q);
+    Hs<T> hp = hess(defp, P), hd = hess(def, P);
     T pxx = hp.xx * dtold, pyy = hp.yy * dtold, pzz = hp.zz * dtold;
     T pxy = hp.xy * dtold, pyz = hp.yz * dtold, pxz = hp.xz * dtold;
     pxx = pxx + hd.xx; pyy = pyy + hd.yy; pzz = pzz + hd.zz;
@@ -178,21 +227,12 @@ __global__ __launch_bounds__(256) void k_complim(T* __restrict__ lim, const T* _
     T cmpmax = cmpmaxglobal * T(1);
     T tlim = T(3) * (T(1) / cmpmax - T(1) / compression) / dtold;
     T v = T(0.);
-    if (tlim > T(0)) { v = tlim; c0 = 1.0; }
-    lim[p] = v;
-    c1 = (double)compression;
+    if (tlim > T(0)) { v = tlim; c0 += 1.0; }
+    P.put(lim, v);
+    c1 = dmax(c1, (double)compression);
   }
-  s[0][threadIdx.x] = c0;
-  s[1][threadIdx.x] = c1;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-      s[0][threadIdx.x] += s[0][threadIdx.x + h];
-      s[1][threadIdx.x] = dmax(s[1][threadIdx.x], s[1][threadIdx.x + h]);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) { bstat[2 * (i64)blockIdx.x] = s[0][0]; bstat[2 * (i64)blockIdx.x + 1] = s[1][0]; }
+  block_stat<0>(c0, part, 0);
+  block_stat<1>(c1, part, 1);
 }
 
 // The compression limiter's correction x (its inverse transform, unnormalised): v = x 2 / n / n / n

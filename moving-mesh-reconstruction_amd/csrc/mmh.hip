@@ -484,12 +484,10 @@ unsigned op_apply(mmh_ctx* c, T* q, double* bres, const T* p, const T* G, int n,
 }
 
 template <class T> void relayout(mmh_ctx* c, T* dst, const T* src, int n, int comps, int to_sl) {
-  const i64 cnt = cube(n) * comps;
-  (void)cnt;
   const i64 n3 = cube(n);
-  for (int f = 0; f < comps; ++f) {  // one field per launch (n^3 <= 2^30 work-items)
-    if (to_sl) k_relayout<T, 1><<<nblk(n3), 256, 0, c->stream>>>(dst + f * n3, src + f * n3, n, 1);
-    else k_relayout<T, 0><<<nblk(n3), 256, 0, c->stream>>>(dst + f * n3, src + f * n3, n, 1);
+  for (int f = 0; f < comps; ++f) {  // one field per launch
+    if (to_sl) k_relayout<T, 1><<<nblk(n3 / 2), 256, 0, c->stream>>>(dst + f * n3, src + f * n3, n);
+    else k_relayout<T, 0><<<nblk(n3 / 2), 256, 0, c->stream>>>(dst + f * n3, src + f * n3, n);
   }
   LAUNCHCHK();
 }
@@ -1004,14 +1002,35 @@ void spectral_inverse(mmh_ctx* c, T* out, const T* spec, T* speq, int n, int mod
   fft_cols<T>(c, z, z, n, (i64)n * n / 2, total, -1, scale);
 }
 
-template <class T> void nsmooth_dev(mmh_ctx* c, T* a, int n, int times) {
-  const i64 n3 = cube(n);
-  T* t = wsT<T>(c, "smooth_tmp", n3);
-  for (int r = 0; r < times; ++r) {
-    k_smooth27<T><<<nblk(n3), 256, 0, c->stream>>>(t, a, n);
-    HIPCHK(hipMemcpyAsync(a, t, sizeof(T) * n3, hipMemcpyDeviceToDevice, c->stream));
-  }
+// One smoothing pass, out of place.
+template <class T> void smooth(mmh_ctx* c, T* out, const T* in, int n) {
+  const unsigned gx = (unsigned)(n * n + 255) / 256;
+  if (n >= 128) k_smooth27<T, 8><<<gx * (n / 8), 256, 0, c->stream>>>(out, in, n);
+  else k_smooth27<T, 4><<<gx * (n / 4), 256, 0, c->stream>>>(out, in, n);  // short walks: more workgroups
   LAUNCHCHK();
+}
+// nsmooth of a, `times` over.
+template <class T> void nsmooth_dev(mmh_ctx* c, T* a, int n, int times) {
+  T* t = wsT<T>(c, "smooth_tmp", cube(n));
+  for (; times >= 2; times -= 2) {
+    smooth(c, t, a, n);
+    smooth(c, a, t, n);
+  }
+  if (times) {
+    smooth(c, t, a, n);
+    HIPCHK(hipMemcpyAsync(a, t, sizeof(T) * cube(n), hipMemcpyDeviceToDevice, c->stream));
+  }
+}
+
+// The nf fields of block results part[f nb + b], each combined by its operation (ops: two bits per field, 0
+// sum of counts, 1 maximum, 2 minimum) on the device, into host values (after a synchronisation).
+template <int NF> void fetch_stats(mmh_ctx* c, const double* part, i64 nb, unsigned ops, double (&out)[NF]) {
+  double* mid = (double*)ws_get(c, "stat_mid", sizeof(double) * NF * 65);
+  k_stats<<<64, 256, 0, c->stream>>>(mid, part, nb, NF, ops);
+  k_stats<<<1, 256, 0, c->stream>>>(mid + 64 * NF, mid, 64, NF, ops);
+  LAUNCHCHK();
+  HIPCHK(hipMemcpyAsync(out, mid + 64 * NF, sizeof(double) * NF, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
 }
 
 template <class T> __global__ void k_pad(T* __restrict__ dst, const T* __restrict__ src, int n, i64 n3) {
@@ -1028,27 +1047,37 @@ template <class T> __global__ void k_pad_speq(T* __restrict__ dst, const T* __re
   dst[(i64)n + 1 + (i64)(n + 2) * r] = sq[2 * r + 1];
 }
 
-// Steps 1-3 of calcdefp: the right-hand side handed to multigrid (limiter.f90:134-392).  hb
-// receives the per-block [nexpand, detmax, detmin, fluxmax, fluxmin] (valid after a sync).
+// Block results of the limiter's kernels, and of k_complim.
+struct LimStatsDev {
+  double* point;  // nexpand, detmax, detmin
+  double* flux;   // fluxmax, fluxmin
+  i64 nb;
+};
+
+// Steps 1-3 of calcdefp: the right-hand side handed to multigrid (limiter.f90:134-392).  rho (may be null)
+// receives the density, made contiguous.
 template <class T>
-void limiter_rhs_dev(mmh_ctx* c, T* tmp, const T* def, const T* u, T dtold, T dtaumesh, int nf, int n, T compressmax,
-                     std::vector<double>& hb, T* gate = nullptr) {
+LimStatsDev limiter_rhs_dev(mmh_ctx* c, T* tmp, const T* def, const T* u, T dtold, T dtaumesh, int nf, int n, T compressmax,
+                            T* gate = nullptr, T* rho = nullptr) {
   const T pi = T(3.14159265358979323846264338328);
   const i64 n3 = cube(n);
-  k_mismatch<T><<<nblk(n3), 256, 0, c->stream>>>(tmp, u, nf, n3, dtold);
+  const unsigned nb = nblk(n3), nl = nblk(n3, 256 * LIM_PT);
+  T* t = wsT<T>(c, "smooth_tmp", n3);
+  T* s3 = wsT<T>(c, "limS3", 3 * n3);
+  unsigned char* flag = (unsigned char*)ws_get(c, "limFlag", (size_t)n3);
+  LimStatsDev st;
+  st.nb = nl;
+  st.point = (double*)ws_get(c, "limstat", sizeof(double) * 5 * nl);
+  st.flux = st.point + 3 * (i64)nl;
+  k_mismatch<T><<<nb, 256, 0, c->stream>>>(t, rho, u, nf, n3, dtold);
+  smooth(c, tmp, t, n);
+  smooth(c, t, tmp, n);
+  smooth(c, tmp, t, n);
+  k_lim_point<T><<<nl, 256, 0, c->stream>>>(s3, flag, def, u, nf, n, dtold, compressmax, pi, st.point);
+  k_eflux<T><<<nl, 256, 0, c->stream>>>(t, tmp, s3, flag, n, dtold, dtaumesh, st.flux, gate);
   LAUNCHCHK();
-  nsmooth_dev(c, tmp, n, 3);
-  T* B = wsT<T>(c, "limB", 7 * n3);
-  k_binv<T><<<nblk(n3), 256, 0, c->stream>>>(B, def, n);
-  T* ef = wsT<T>(c, "limE", n3);
-  const unsigned nb = nblk(n3);
-  double* bst = (double*)ws_get(c, "limstat", sizeof(double) * 5 * nb);
-  k_eflux<T><<<nb, 256, 0, c->stream>>>(ef, tmp, B, def, u, nf, n, dtold, dtaumesh, compressmax, pi, bst, gate);
-  LAUNCHCHK();
-  hb.assign(5 * (size_t)nb, 0.0);
-  HIPCHK(hipMemcpyAsync(hb.data(), bst, sizeof(double) * hb.size(), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(tmp, ef, sizeof(T) * n3, hipMemcpyDeviceToDevice, c->stream));
-  nsmooth_dev(c, tmp, n, 1);
+  smooth(c, tmp, t, n);
+  return st;
 }
 
 void solve_dev(mmh_ctx* c, double* u, double* rhs, const double* defpot, const double* ubig, int n, int nu,
@@ -1088,25 +1117,22 @@ void calcdefp_dev(mmh_ctx* c, T* defp, T* tmp, T* tmp2, const T* def, const T* u
   if (ng <= 0) ng = n;
   const T pi = T(3.14159265358979323846264338328);
   const i64 n3 = cube(n);
-  std::vector<double> hb;
-  limiter_rhs_dev<T>(c, tmp, def, u, dtold, dtaumesh, nf, n, compressmax, hb);
+  T* rho = wsT<T>(c, "limRho", n3);
+  const LimStatsDev ls = limiter_rhs_dev<T>(c, tmp, def, u, dtold, dtaumesh, nf, n, compressmax, (T*)nullptr, rho);
   fill<T>(c, defp, T(0), n3);
   mmh_mg_stats* mst = st ? &st->mg : nullptr;
-  if (c->mesh_solve) mesh_solve_dev(c, defp, tmp, def, u, n, nf, ng);
-  else multigrid_dev<T>(c, defp, tmp, def, u, T(1.), n, nf, 2, ng, mst);
+  if (c->mesh_solve) mesh_solve_dev(c, defp, tmp, def, rho, n, 1, ng);
+  else multigrid_dev<T>(c, defp, tmp, def, rho, T(1.), n, 1, 2, ng, mst);
   nsmooth_dev(c, defp, n, 2);
-  const unsigned nb = nblk(n3);
   T* lim = wsT<T>(c, "limL", n3);
+  const unsigned nl = nblk(n3, 256 * LIM_PT);
+  double* bst2 = (double*)ws_get(c, "limstat2", sizeof(double) * 2 * nl);
+  k_complim<T><<<nl, 256, 0, c->stream>>>(lim, defp, def, n, dtold, compressmax, pi, bst2);
   LAUNCHCHK();
-  double* bst2 = (double*)ws_get(c, "limstat2", sizeof(double) * 2 * nb);
-  k_complim<T><<<nb, 256, 0, c->stream>>>(lim, defp, def, n, dtold, compressmax, pi, bst2);
-  LAUNCHCHK();
-  std::vector<double> hb2(2 * (size_t)nb);
-  HIPCHK(hipMemcpyAsync(hb2.data(), bst2, sizeof(double) * hb2.size(), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  long ncompress = 0;
-  double cmax = 0;
-  for (unsigned b = 0; b < nb; ++b) { ncompress += (long)hb2[2 * b]; cmax = std::max(cmax, hb2[2 * b + 1]); }
+  double hc[2];  // ncompress, cmax
+  fetch_stats<2>(c, bst2, nl, 0u | 1u << 2, hc);
+  const long ncompress = (long)hc[0];
+  const double cmax = std::max(0.0, hc[1]);
   if (ncompress > 0) {
     T* sq = wsT<T>(c, "limS", 2 * (i64)n * n);
     C2<T>* z = reinterpret_cast<C2<T>*>(lim);
@@ -1121,20 +1147,16 @@ void calcdefp_dev(mmh_ctx* c, T* defp, T* tmp, T* tmp2, const T* def, const T* u
   // exit convention of tmp (limiter.f90:621-628,669-671): all cells "hot" -> 1; diagnostics 0
   fill<T>(c, tmp, T(1), n3);
   fill<T>(c, tmp, T(0), 3);
-  HIPCHK(hipStreamSynchronize(c->stream));
   if (st) {
-    double detmax = 0, detmin = 1, fmaxv = 0, fminv = 0;
-    long nexp = 0;
-    for (unsigned b = 0; b < nb; ++b) {
-      nexp += (long)hb[5 * b];
-      detmax = std::max(detmax, hb[5 * b + 1]);
-      detmin = std::min(detmin, hb[5 * b + 2]);
-      fmaxv = std::max(fmaxv, hb[5 * b + 3]);
-      fminv = std::min(fminv, hb[5 * b + 4]);
-    }
-    st->cmax = cmax; st->detmin = detmin; st->detmax = detmax; st->fluxmin = fminv; st->fluxmax = fmaxv;
-    st->nexpand = (int)nexp; st->ncompress = (int)ncompress;
+    double hp[3], hf[2];  // nexpand, detmax, detmin; fluxmax, fluxmin
+    fetch_stats<3>(c, ls.point, ls.nb, 0u | 1u << 2 | 2u << 4, hp);
+    fetch_stats<2>(c, ls.flux, ls.nb, 1u | 2u << 2, hf);
+    st->cmax = cmax;
+    st->detmax = std::max(0.0, hp[1]); st->detmin = std::min(1.0, hp[2]);
+    st->fluxmax = std::max(0.0, hf[0]); st->fluxmin = std::min(0.0, hf[1]);
+    st->nexpand = (int)(long)hp[0]; st->ncompress = (int)ncompress;
   }
+  HIPCHK(hipStreamSynchronize(c->stream));
 }
 
 template <class T> void relaxing_dev(mmh_ctx* c, T* u, const T* def, const T* defp, T dt, int nf, int n) {
@@ -1919,8 +1941,7 @@ void recon_power_dev(mmh_ctx* c, const double* rho, const double* defin, int n, 
   }
   // forward: rhs (gates recorded), its sum (rgzerosum's), solve, defp = S^2 phi, compression
   // check, delta = D(def + defp), binned power
-  std::vector<double> hb;
-  limiter_rhs_dev<double>(c, rhs, d0, u, 1.0, 1.0, 5, n, 10.0, hb, gate);
+  limiter_rhs_dev<double>(c, rhs, d0, u, 1.0, 1.0, 5, n, 10.0, gate);
   reduce<double>(c, rhs, n3, 0, sums + 0);  // sum r
   k_det<double><<<nblk(n3), 256, 0, c->stream>>>(det, d0, n, 1.0);
   LAUNCHCHK();
@@ -1930,19 +1951,17 @@ void recon_power_dev(mmh_ctx* c, const double* rho, const double* defin, int n, 
   o.tol = tol; o.max_cycles = 256; o.schedule = 1; o.nu_pre = 2; o.nu_post = 2; o.nu_coarse = 8; o.ng = 0;
   o.mixed = 0; o.krylov = 1;
   mmh_solve_stats s1;
-  solve_dev(c, phi, rhs, d0, u, n, 5, &o, &s1);
+  solve_dev(c, phi, rhs, d0, rho, n, 1, &o, &s1);
   HIPCHK(hipMemcpyAsync(w1, phi, sizeof(double) * n3, hipMemcpyDeviceToDevice, c->stream));
   nsmooth_dev<double>(c, w1, n, 2);
-  const unsigned nbk = nblk(n3);
+  const unsigned nbk = nblk(n3, 256 * LIM_PT);
   double* lim = wsT<double>(c, "ad_lim", n3);
   double* bst = (double*)ws_get(c, "ad_limstat", sizeof(double) * 2 * nbk);
   k_complim<double><<<nbk, 256, 0, c->stream>>>(lim, w1, d0, n, 1.0, 10.0, pi, bst);
   LAUNCHCHK();
-  std::vector<double> hc(2 * (size_t)nbk);
-  HIPCHK(hipMemcpyAsync(hc.data(), bst, sizeof(double) * hc.size(), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  long ncomp = 0;
-  for (unsigned b = 0; b < nbk; ++b) ncomp += (long)hc[2 * b];
+  double hc[2];
+  fetch_stats<2>(c, bst, nbk, 0u | 1u << 2, hc);
+  const long ncomp = (long)hc[0];
   if (st) {
     std::memset(st, 0, sizeof(*st));
     st->cycles_forward = s1.cycles;
@@ -1986,7 +2005,7 @@ void recon_power_dev(mmh_ctx* c, const double* rho, const double* defin, int n, 
   double* lam = dl;
   fill<double>(c, lam, 0.0, n3);
   mmh_solve_stats s2;
-  solve_dev(c, lam, rhs, d0, u, n, 5, &o, &s2);
+  solve_dev(c, lam, rhs, d0, rho, n, 1, &o, &s2);
   if (st) {
     st->cycles_adjoint = s2.cycles;
     st->relres_adjoint = s2.cycles > 0 ? s2.relres[s2.cycles - 1] : 0.0;
@@ -2409,8 +2428,7 @@ int mmh_limiter_rhs_d(mmh_ctx* c, double* tmp, const double* def, const double* 
   return guarded(c, [&] {
     require(is_pow2(n) && n >= 16 && n <= 1024 && nf >= 4, "limiter_rhs: bad size");
     require(compressmax >= 0, "limiter_rhs: compressmax < 0");
-    std::vector<double> hb;
-    limiter_rhs_dev<double>(c, tmp, def, u, dtold < 1.e-8 ? 1.0 : dtold, dtaumesh, nf, n, compressmax, hb);
+    limiter_rhs_dev<double>(c, tmp, def, u, dtold < 1.e-8 ? 1.0 : dtold, dtaumesh, nf, n, compressmax);
     HIPCHK(hipStreamSynchronize(c->stream));
   });
 }
