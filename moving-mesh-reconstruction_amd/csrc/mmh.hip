@@ -457,12 +457,24 @@ unsigned march_op(mmh_ctx* c, T* out, double* bres, const T* phi, const T* rhs, 
   }
 }
 
+// Levels whose residual is formed a thread per point (k_resid_pt): those the k-marching kernel does not take
+// (n < 64), and 64^3 by itself or in pairs.  128^3 is faster marched (31 against 50 us in FP64).
+inline bool resid_pt(int n, int B) { return n < 64 || (n == 64 && B <= 2); }
+// Block results of op_resid at most, per grid.
+inline unsigned resid_blocks(int n) { return n <= 64 ? nblk(cube(n), RB) : stencil_grid(n, 1); }
+
 // r = rhs - L phi on a sub-lattice level (r may be null) with per-block max|r| into bres, for B
 // grids stored one after another when batched (act: grids y with act[y] = 0 are skipped); returns
 // the number of block results per grid.
 template <class T, class TG = T>
 unsigned op_resid(mmh_ctx* c, T* r, double* bres, const T* phi, const T* rhs, const TG* G, int n, T di2,
                   bool delta = false, int B = 1, int batched = 0, const int* act = nullptr) {
+  if (!delta && resid_pt(n, B)) {
+    const unsigned nb = nblk(cube(n), RB);
+    k_resid_pt<T, TG><<<dim3(nb, B), RB, 0, c->stream>>>(r, bres, phi, rhs, G, n, di2, batched, act);
+    LAUNCHCHK();
+    return nb;
+  }
   if (!delta)
     if (const unsigned nb = march_op<T, 0, TG>(c, r, bres, phi, rhs, G, n, di2, B, batched, act)) return nb;
   const unsigned nb = stencil_grid(n, 1);
@@ -560,20 +572,25 @@ template <class F> void colour_steps(int ns, bool reverse, bool pairs, bool from
     }
 }
 
-// ns 19-point sweeps of a 32^3 level tile by tile, one launch per sweep (k_sweep_tile), between phi and a
-// second buffer; the result ends in phi.
+// ns sweeps of a 32^3 level tile by tile, one launch per sweep (k_sweep_tile from the metric, or with GAL
+// k_sweep_tile_gal from Galerkin coefficients), between phi and a second buffer; the result ends in phi.
 constexpr int TILE_N = 32;
-template <class T, class TG>
+template <bool GAL, class T, class TG>
 void tile_sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* G, int n, T dx2, int ns, bool reverse) {
   if (ns < 1) return;
-  constexpr int TK = 2;
+  constexpr int TK = 2, NT = TileShape<TK, GAL>::NT;
   T* tmp = wsT<T>(c, "tile_tmp", cube(TILE_N));
   const unsigned nb = (unsigned)((n / 8) * (n / 8) * (n / TK));
   T* src = phi;
   T* dst = tmp;
   for (int s = 0; s < ns; ++s) {
-    if (reverse) k_sweep_tile<T, TG, true, TK><<<nb, TileShape<TK>::NT, 0, c->stream>>>(dst, src, rhs, G, n, dx2);
-    else k_sweep_tile<T, TG, false, TK><<<nb, TileShape<TK>::NT, 0, c->stream>>>(dst, src, rhs, G, n, dx2);
+    if constexpr (GAL) {
+      if (reverse) k_sweep_tile_gal<T, TG, true, TK><<<nb, NT, 0, c->stream>>>(dst, src, rhs, G, n);
+      else k_sweep_tile_gal<T, TG, false, TK><<<nb, NT, 0, c->stream>>>(dst, src, rhs, G, n);
+    } else {
+      if (reverse) k_sweep_tile<T, TG, true, TK><<<nb, NT, 0, c->stream>>>(dst, src, rhs, G, n, dx2);
+      else k_sweep_tile<T, TG, false, TK><<<nb, NT, 0, c->stream>>>(dst, src, rhs, G, n, dx2);
+    }
     std::swap(src, dst);
   }
   if (src != phi) k_copy_strided<T><<<nblk(cube(n)), 256, 0, c->stream>>>(phi, src, cube(n), 1);
@@ -602,7 +619,7 @@ void sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* G, int n, T dx, int ns, 
   }
   const int S = (layout == 1 && n >= c->colour_col_min_n && h % c->colour_col == 0) ? c->colour_col : 1;
   if (layout == 1 && !delta && S == 1 && n == TILE_N) {
-    tile_sweeps<T, TG>(c, phi, rhs, G, n, dx2, ns, reverse);
+    tile_sweeps<false, T, TG>(c, phi, rhs, G, n, dx2, ns, reverse);
     return;
   }
   if (c->slab_now > 1 && S == 8 && !delta && n >= 512 && (h / S) % c->slab_now == 0) {
@@ -650,7 +667,7 @@ void relax_dev(mmh_ctx* c, T* phi, const T* rhs, const TG* G, T* rscratch, int n
                double* rinf_dev, bool reverse = false, bool delta = false, bool from_zero = false) {
   sweeps<T, TG>(c, phi, rhs, G, n, dx, nrelax, 1, reverse, delta, from_zero);
   if (!want_norm && !rc) return;
-  double* bmax = (double*)ws_get(c, "bmax", sizeof(double) * stencil_grid(n, 1));
+  double* bmax = (double*)ws_get(c, "bmax", sizeof(double) * resid_blocks(n));
   const unsigned nb = op_resid<T, TG>(c, rc ? rscratch : nullptr, bmax, phi, rhs, G, n, T(1) / (dx * dx), delta);
   if (want_norm) reduce<double>(c, bmax, nb, 1, rinf_dev);
   if (rc) {
@@ -665,6 +682,10 @@ void relax_dev(mmh_ctx* c, T* phi, const T* rhs, const TG* G, T* rscratch, int n
 // residual stored in r and restricted into rc with calcresid's plane order rule.
 template <class T, class TG = T>
 void gal_sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* A, int n, int ns, bool reverse, bool from_zero = false) {
+  if (n == TILE_N) {
+    tile_sweeps<true, T, TG>(c, phi, rhs, A, n, T(0), ns, reverse);
+    return;
+  }
   const unsigned nb = nblk(cube(n / 2));
   for (int s = 0; s < ns; ++s)
     for (int cc = 0, done = 0; cc < 8; ++cc) {
@@ -1833,8 +1854,7 @@ void solve_dev(mmh_ctx* c, double* u, double* rhs, const double* defpot, const d
   Hier<float> F;
   build_fp32(c, F, H);
   double* r64 = H.r[0];
-  const unsigned nb = stencil_grid(n, 1);
-  double* bmax = (double*)ws_get(c, "sbmax", sizeof(double) * nb);
+  double* bmax = (double*)ws_get(c, "sbmax", sizeof(double) * resid_blocks(n));
   for (int cyc = 0; cyc < o->max_cycles; ++cyc) {
     op_resid<double>(c, r64, bmax, us, rs, H.G[0], n, 1.0);
     k_convert<double, float><<<nblk(n3), 256, 0, c->stream>>>(F.rhs[0], r64, n3);
