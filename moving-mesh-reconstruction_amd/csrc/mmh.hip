@@ -597,6 +597,22 @@ void tile_sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* G, int n, T dx2, in
   LAUNCHCHK();
 }
 
+// Half-sweep slabs.  A point's 19-point neighbours in the other k parity are never updated in its
+// own half sweep (four colours), and those of its own parity lie in its own plane: planes are
+// independent inside a half sweep, so the four colours can follow one another on a slab of planes
+// before the next slab, with the values of the colour-by-colour order.  The slab's eight class
+// arrays then stay in the 256 MB Infinity Cache between its launches.  The line: FP32 values and
+// coefficients from 512^3, 2250 -> 2030 us a sweep there, 17.0 -> 15.0 ms at 1024^3; at 256^3 the
+// level fits the cache whole and the extra launches cost (220 -> 245 us), and FP64 sweeps gain
+// nothing in any slab size (4620 us against 4640 to 9420).  A slab is the smallest that still
+// gives 512 workgroups: 16 planes of a class at 512^3 (32 planes: 2040 to 2200 us, 8 planes: 2680),
+// 8 at 1024^3 (16 and 32 planes: 17.0 ms).
+constexpr int HALF_SLAB_MIN_N = 512;
+static int half_slab_per(int n) {
+  const int nb = (int)colour_col_blocks(n);
+  return std::max(1, (511 + nb) / nb);
+}
+
 // from_zero: phi is 0 on entry, so the first sweep's colours read only the classes updated before
 // them in that sweep (k_colour's MASK form; same values).
 template <class T, class TG = T>
@@ -640,6 +656,23 @@ void sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* G, int n, T dx, int ns, 
                                                                         col & 1, 0xFFu, b * per, per);
         }
       }
+    LAUNCHCHK();
+    return;
+  }
+  if constexpr (std::is_same<T, float>::value && std::is_same<TG, float>::value)
+  if (S == 8 && !delta && !from_zero && n >= HALF_SLAB_MIN_N) {
+    // FP32 sweeps from a value: the four colours of one k parity, slab by slab (half_slab_per)
+    const int nz = h / S, per = half_slab_per(n);
+    const unsigned nbs = colour_col_blocks(n) * (unsigned)per;
+    require(nz % per == 0, "sweeps: a slab must divide the segments of a class");
+    for (int s = 0; s < ns; ++s)
+      for (int half = 0; half < 2; ++half)
+        for (int b = 0; b < nz; b += per)
+          for (int cc = 4 * half; cc < 4 * half + 4; ++cc) {
+            const int col = reverse ? 7 - cc : cc;
+            k_colour_col<T, false, false, 8, TG><<<nbs, 256, 0, c->stream>>>(phi, rhs, G, n, dx2, col >> 2, (col >> 1) & 1,
+                                                                          col & 1, 0xFFu, b, per);
+          }
     LAUNCHCHK();
     return;
   }

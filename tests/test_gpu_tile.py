@@ -45,6 +45,25 @@ def test_bfloat16_tile_sweeps_equal_the_oracle(ctx, ns):
     assert np.array_equal(got.cpu().numpy(), phi)
 
 
+@pytest.mark.parametrize("n", [512, 1024])
+def test_half_sweep_slabs_equal_the_colour_by_colour_order(ctx, n):
+    """FP32 sweeps from 512^3 go slab by slab inside a half sweep (two segments of 8 planes a slab, one at
+    1024^3); one point per thread (option colour_col = 1) goes colour by colour.  Equality."""
+    print("case half-sweep slabs n=%d" % n, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    draw = lambda k: torch.rand(k, device="cuda", generator=gen)  # noqa: E731
+    rhs, G = draw(n ** 3) - 0.5, draw(6 * n ** 3) + 1.0
+    a = draw(n ** 3)
+    b = a.clone()
+    ctx.time_sweeps(a, rhs, G, 1.0, 2)
+    try:
+        ctx.set_option("colour_col", 1)
+        ctx.time_sweeps(b, rhs, G, 1.0, 2)
+    finally:
+        ctx.set_option("colour_col", 8)
+    assert bool(torch.isfinite(a).all()) and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("mixed", [0, 1])
 @pytest.mark.parametrize("nu", [1, 2, 3])
 def test_galerkin_tile_sweeps_inside_a_solve(ctx, mixed, nu):
