@@ -230,9 +230,27 @@ __device__ __forceinline__ T gal_resid_point(const T* __restrict__ phi, const T*
 // qi + h qj + h^2 qk); Ac = A + c h^3 (the point's class in each coefficient field), h a power of two.
 // TG = bf16x2: the 27 fields in 14 words (fields 2f, 2f + 1 in word f), read as words.  The centre
 // coefficient comes back in a13.
-template <class T, bool MASK, class TG>
-__device__ __forceinline__ T gal_offsum_cls(const T* __restrict__ phi, const TG* __restrict__ Ac, int h, int c, int qi,
-                                           int qj, int qk, unsigned o0, unsigned live, T& a13) {
+// PAIR: without the values of the two neighbours along j (fields 10 and 16).
+template <class T, bool MASK, class TG, bool PAIR = false> struct GalTerms {
+  T av[27], vv[27], a13;
+  bool use[27];
+  __device__ __forceinline__ void load(const T* __restrict__ phi, const TG* __restrict__ Ac, int h, int c, int qi, int qj,
+                                       int qk, unsigned o0, unsigned live);
+  __device__ __forceinline__ T sum() const {
+    T s = T(0);
+#pragma unroll
+    for (int e = 0; e < 27; ++e) {
+      if (e == 13) continue;
+      if (MASK && !use[e]) continue;
+      s = s + av[e] * vv[e];
+    }
+    return s;
+  }
+};
+template <class T, bool MASK, class TG, bool PAIR>
+__device__ __forceinline__ void GalTerms<T, MASK, TG, PAIR>::load(const T* __restrict__ phi, const TG* __restrict__ Ac, int h,
+                                                                 int c, int qi, int qj, int qk, unsigned o0,
+                                                                 unsigned live) {
   const int hm = h - 1;
   const i64 h3 = (i64)h * h * h, n3 = 8 * h3;
   const int io = c & 1, jo = (c >> 1) & 1, ko = c >> 2;
@@ -248,8 +266,6 @@ __device__ __forceinline__ T gal_offsum_cls(const T* __restrict__ phi, const TG*
   // All loads first, then the sum.  With MASK a left-out term still loads, from the point's own
   // centre coefficient and value (read by the update anyway, so no extra memory traffic), and is
   // skipped in the sum: loads behind a branch would each be waited for before the next.
-  T av[27], vv[27];
-  bool use[27];
   use[13] = false;
 #pragma unroll
   for (int e = 0; e < 27; ++e) {
@@ -257,6 +273,7 @@ __device__ __forceinline__ T gal_offsum_cls(const T* __restrict__ phi, const TG*
     const int ex = e % 3 - 1, ey = (e / 3) % 3 - 1, ez = e / 9 - 1;
     use[e] = !MASK || ((live >> (cc ^ (4u * (ez != 0) + 2u * (ex != 0) + (ey != 0)))) & 1u);
     const int cn = use[e] ? c ^ ((ex != 0) | ((ey != 0) << 1) | ((ez != 0) << 2)) : c;
+    if (PAIR && (e == 10 || e == 16)) continue;
     const unsigned on = use[e] ? X[ex + 1] + Y[ey + 1] + Z[ez + 1] : o0;
     vv[e] = *(const T*)((const char*)(phi + (i64)cn * h3) + (uint32_t)(on * (unsigned)sizeof(T)));
   }
@@ -282,14 +299,14 @@ __device__ __forceinline__ T gal_offsum_cls(const T* __restrict__ phi, const TG*
     }
     a13 = gl<T>((const TG*)((const char*)(Ac + 13 * n3) + (uint32_t)(o0 * (unsigned)sizeof(TG))), 0);
   }
-  T s = T(0);
-#pragma unroll
-  for (int e = 0; e < 27; ++e) {
-    if (e == 13) continue;
-    if (MASK && !use[e]) continue;
-    s = s + av[e] * vv[e];
-  }
-  return s;
+}
+template <class T, bool MASK, class TG>
+__device__ __forceinline__ T gal_offsum_cls(const T* __restrict__ phi, const TG* __restrict__ Ac, int h, int c, int qi,
+                                           int qj, int qk, unsigned o0, unsigned live, T& a13) {
+  GalTerms<T, MASK, TG> P;
+  P.load(phi, Ac, h, c, qi, qj, qk, o0, live);
+  a13 = P.a13;
+  return P.sum();
 }
 
 // Batched launches: gridDim.y = B grids stored one after another (bstride = n^3 values; A holds
@@ -317,6 +334,45 @@ __global__ __launch_bounds__(256) void k_gal_colour(T* __restrict__ phi, const T
   T a13;
   const T s = gal_offsum_cls<T, MASK, TG>(phi, Ac, h, c, qi, qj, qk, (unsigned)q, live, a13);
   *pc = (rv - s) / a13;
+}
+
+// Two colours of a 64^3 level in one launch: (k, i, j0) and the one after it, which differs in the parity
+// of j alone.  The two are coupled only along j, and a workgroup holds GAL_PAIR_W whole lines of a class
+// along j, so it updates the first colour, passes it through LDS, and updates the second, whose other
+// operands are loaded before the barrier; no workgroup reads what another one of the launch writes.
+// Products are summed in the same order: the values are those of the two launches.
+// A launch is bound by its latency, not by its bytes: registers for both colours' operands in flight, and
+// as many workgroups as compute units.  FP64, per sweep: 36 us colour by colour, 22.5 us with lines of 4
+// points side by side (256 workgroups); 2: 34, 8: 26, 16: 35.  Only 64^3: 32^3 is swept in one launch,
+// and from 128^3 a colour's own bytes are the cost and lines of 64 points would shorten its loads.
+constexpr int GAL_PAIR_N = 64, GAL_PAIR_W = 4;
+template <class T, bool MASK = false, class TG = T>
+__global__ __launch_bounds__(GAL_PAIR_N / 2 * GAL_PAIR_W) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_gal_pair(T* __restrict__ phi, const T* __restrict__ rhs,
+                                                                         const TG* __restrict__ A, int kpar, int io,
+                                                                         int j0, unsigned live = 0xFFu) {
+  constexpr int H = GAL_PAIR_N / 2, W = GAL_PAIR_W;
+  constexpr i64 h3 = (i64)H * H * H;
+  __shared__ T u[H * W];
+  const int blk = (int)xcd_remap(blockIdx.x, gridDim.x), t = threadIdx.x;
+  const int qi = W * (blk % (H / W)) + t % W, qj = t / W, qk = blk / (H / W);
+  const unsigned o0 = (unsigned)(qi + H * qj + H * H * qk);
+  const uint32_t ob = o0 * (uint32_t)sizeof(T);
+  const int c1 = io | (j0 << 1) | (kpar << 2), c2 = c1 ^ 2;
+  GalTerms<T, MASK, TG> P;
+  GalTerms<T, MASK, TG, true> Q;
+  P.load(phi, A + (i64)c1 * h3, H, c1, qi, qj, qk, o0, live);
+  Q.load(phi, A + (i64)c2 * h3, H, c2, qi, qj, qk, o0, live | 1u << (4 * kpar + 2 * io + j0));
+  T* p1 = (T*)((char*)(phi + (i64)c1 * h3) + ob);
+  T* p2 = (T*)((char*)(phi + (i64)c2 * h3) + ob);
+  const T r1 = *(const T*)((const char*)(rhs + (i64)c1 * h3) + ob), r2 = *(const T*)((const char*)(rhs + (i64)c2 * h3) + ob);
+  const T v1 = (r1 - P.sum()) / P.a13;
+  u[t] = v1;
+  *p1 = v1;
+  __syncthreads();
+  // the second colour's neighbours at j - 1 and j + 1: its own line of the first, one entry up or down
+  Q.vv[10] = u[j0 ? (qj + H - 1) % H * W + t % W : t];
+  Q.vv[16] = u[j0 ? t : (qj + 1) % H * W + t % W];
+  *p2 = (r2 - Q.sum()) / Q.a13;
 }
 
 // Workgroups of k_gal_resid for an n^3 level: gal_resid_blocks(n) / 8 per sub-lattice class.

@@ -719,6 +719,20 @@ void gal_sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* A, int n, int ns, bo
     tile_sweeps<true, T, TG>(c, phi, rhs, A, n, T(0), ns, reverse);
     return;
   }
+  if (n == GAL_PAIR_N) {
+    // colours two by two (k_gal_pair)
+    constexpr unsigned nbp = GAL_PAIR_N / 2 * GAL_PAIR_N / 2 / GAL_PAIR_W, nt = GAL_PAIR_N / 2 * GAL_PAIR_W;
+    for (int s = 0; s < ns; ++s)
+      for (int cc = 0, done = 0; cc < 8; cc += 2) {
+        const int col = reverse ? 7 - cc : cc;
+        if (s == 0 && from_zero)
+          k_gal_pair<T, true, TG><<<nbp, nt, 0, c->stream>>>(phi, rhs, A, col >> 2, (col >> 1) & 1, col & 1, (unsigned)done);
+        else k_gal_pair<T, false, TG><<<nbp, nt, 0, c->stream>>>(phi, rhs, A, col >> 2, (col >> 1) & 1, col & 1);
+        done |= 1 << col | 1 << (col ^ 1);
+      }
+    LAUNCHCHK();
+    return;
+  }
   const unsigned nb = nblk(cube(n / 2));
   for (int s = 0; s < ns; ++s)
     for (int cc = 0, done = 0; cc < 8; ++cc) {

@@ -45,6 +45,32 @@ def test_bfloat16_tile_sweeps_equal_the_oracle(ctx, ns):
     assert np.array_equal(got.cpu().numpy(), phi)
 
 
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("nu", [1, 2])
+def test_paired_galerkin_colours_inside_a_solve(ctx, mixed, nu):
+    """A 128^3 Krylov solve sweeps its 64^3 Galerkin level two colours a launch, from zero and from a
+    value, forward and reversed: the FP64 solve equals the batched one, which sweeps colour by colour;
+    the mixed one (bfloat16 coefficients) reaches the tolerance under the FP64 operator."""
+    print("case galerkin pairs mixed=%d nu=%d" % (mixed, nu), flush=True)
+    n = 128
+    rng = np.random.default_rng(nu)
+    u = np.zeros((n ** 3, 5))
+    u[:, 0] = R.or_lognormal(n, 1.5, 3)
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a).ravel()).cuda()  # noqa: E731
+    rhs, ud, d = rng.standard_normal(n ** 3), to(u), to(np.zeros(n ** 3))
+    phi, b = to(np.zeros(n ** 3)), to(rhs)
+    _, ok = ctx.solve(phi, b, d, ud, tol=1e-9, max_cycles=200, schedule=1, nu_pre=nu, nu_post=nu, nu_coarse=4,
+                      mixed=mixed, nu=5, krylov=True)
+    assert ok
+    if not mixed:
+        phi2, b2 = to(np.zeros(n ** 3)), to(rhs)
+        _, ok2 = ctx.solve_batch([(phi2, b2, d, ud)], tol=1e-9, max_cycles=200, nu_pre=nu, nu_coarse=4, nu=5)
+        assert ok2 and np.array_equal(phi.cpu().numpy(), phi2.cpu().numpy())
+    r = torch.zeros_like(b)
+    ctx.residual(r, phi, b, d, ud)
+    assert float(r.abs().max()) <= 1.01e-9 * float(b.abs().max())
+
+
 @pytest.mark.parametrize("n", [512, 1024])
 def test_half_sweep_slabs_equal_the_colour_by_colour_order(ctx, n):
     """FP32 sweeps from 512^3 go slab by slab inside a half sweep (two segments of 8 planes a slab, one at
