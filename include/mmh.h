@@ -131,8 +131,8 @@ int mmh_release_workspace(mmh_ctx* ctx);            /* free cached device buffer
  *                 r and r_old rounded to FP32 (as its FP32 preconditioner receives r) and keeps
  *                 r_old in FP32 only, and the same pass forms the sum of z that removes its mean;
  *                 the residual recurrence and the stopping test stay FP64
- *   "coarse_lds"  1 (default) / 0: the one-workgroup cycle holds its smallest levels (u, rhs, G)
- *                 in LDS while it runs (bit-identical)
+ *   "coarse_lds"  1 (default) / 0: the one-workgroup cycle holds its levels on chip while it runs
+ *                 (16^3 and below: iterate in LDS, coefficients in registers; bit-identical)
  *   "sweep_slabs" 4 (default), 2, 8, 16, 32 or 0: the mixed solve's finest-level sweeps (n >= 512)
  *                 run all colours on one k-slab before the next (this many slabs; the reverse
  *                 sweep in exactly reverse order).  Another Gauss-Seidel order: the preconditioner

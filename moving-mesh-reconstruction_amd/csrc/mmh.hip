@@ -56,7 +56,7 @@ struct mmh_ctx {
   int coarse_fused = 16;   // Krylov preconditioner: levels <= this size in one workgroup (option "coarse_fused", 0 off)
   int sweep_slabs = 4;  // mixed preconditioner's finest level (n >= 512): colour sweeps slab by slab (option "sweep_slabs", 0 off)
   int slab_now = 0;     // set while such sweeps are issued
-  int coarse_lds = 1;      // one-workgroup coarse cycle: its smallest levels held in LDS (option "coarse_lds")
+  int coarse_lds = 1;      // one-workgroup coarse cycle: its levels held on chip (option "coarse_lds")
   int dots32 = 1;          // mixed Krylov solve: z.r and z.r_old from the FP32 roundings of r (option "dots32")
   int coarse_fused_ref = 16;  // the reference V-cycle's levels <= this size in one workgroup (option "coarse_fused_ref")
   int zero_start = 1;      // first sweep from u = 0 reads only the colour classes already updated (option "zero_start")
@@ -762,8 +762,8 @@ void gal_relax(mmh_ctx* c, T* phi, const T* rhs, const TG* A, T* r, int n, int n
 // operators too; at 32^3 a level's sweeps move megabytes through one CU and the launches win).
 // The reference schedule (kind 0: guard, nu = 4 NG/N) fuses its 19-point levels up to the size set
 // by option "coarse_fused_ref" (16 by default: the 16^3..4^3 levels run 128, 256 and 32+32 sweeps,
-// some 3000 launches per V-cycle otherwise; at 512^3 both take 88-89 ms per cycle, and fusing 32^3
-// as well is slower, one CU then carrying the 32^3 level).
+// some 3000 launches per V-cycle otherwise, or 1.2 ms in one workgroup at NG = 512; fusing 32^3 as well
+// is slower, one CU then carrying the 32^3 level).
 template <class T> bool coarse_cycle_applies(const mmh_ctx* c, const Hier<T>& H, int l, const Sched& S) {
   if (S.delta || H.nlev - l > CLEV_MAX) return false;
   for (int q = l; q < H.nlev; ++q)
