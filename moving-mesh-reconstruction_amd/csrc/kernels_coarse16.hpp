@@ -17,28 +17,61 @@
 // 6 phases per sweep instead of 8, the same values.
 // The per-point arithmetic, the order of every sum and the schedule are cw_cycle's, so results are
 // bit-identical.  Measured (MI355X), per cycle: FP32 reference schedule 1124 -> 244 us at NG = 64 and
-// 5.87 -> 1.22 ms at NG = 512 (0.24 us per phase); FP64 Krylov schedule with Galerkin levels 408 -> 124 us;
-// in a batch, one workgroup per grid, 614 -> 126 us.
+// 5.87 -> 1.22 ms at NG = 512 (0.24 us per phase); FP64 Krylov schedule with Galerkin levels 408 -> 127 us;
+// in a batch, one workgroup per grid, 614 -> 128 us.
 #pragma once
+#include <limits>
+
 #include "kernels_coarse.hpp"
 
 namespace mmh {
 
 // a / b for y = 1 / b rounded to nearest: two residual corrections give the correctly rounded
 // quotient (P. Markstein, IBM J. Res. Dev. 34, 1990), 5 dependent operations where the compiler's
-// division takes 11; div_fixup gives zeros, infinities and NaN their IEEE results.  (Exact while the
-// residuals do not underflow, |a| > 2^-100 in FP32.)
-__device__ __forceinline__ float quotient(float a, float b, float y) {
-  float q = a * y;
-  q = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
-  q = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
-  return __builtin_amdgcn_div_fixupf(q, b, a);
+// division takes 11; div_fixup gives zeros, infinities and NaN their IEEE results.  It is exact while y, the
+// quotient and the residuals stay normal numbers: in FP32 |a| from 2^-100 (the residual is a multiple of 2^-47
+// |a|, and 2^-149 the smallest step), |b| and |q| from 2^-126, |b| up to 2^126.  The bounds kept here, |a| from
+// 2^-80 and |b| up to 2^44 (FP64 2^-600, 2^400), make |q| large enough too.  A Range holds the
+// smallest dividend but zero of a thread, in two integer operations a quotient; where it or a divisor is out
+// of bounds, or the iterate is not finite (a quotient that overflows leaves it so), the cycle is run
+// again by the general form, whose divisions are plain.  A test on every quotient that chose the
+// division there cost 9 % of the FP32 cycle, flags of three comparisons 6 %.
+struct Range {
+  unsigned key = ~0u;  // of the smallest dividend: its bits without the sign, less one
+  static __device__ __forceinline__ unsigned key_of(float a) { return (__float_as_uint(a) << 1) - 1u; }
+  static __device__ __forceinline__ unsigned key_of(double a) {  // of the high word; one more below it if the low is set
+    return ((unsigned)__double2hiint(a) << 1) + min((unsigned)__double2loint(a), 1u) - 1u;
+  }
+  template <class T> __device__ __forceinline__ void dividend(T a) { key = min(key, key_of(a)); }
+  __device__ __forceinline__ void divisor(float b) {
+    if (!(fabs(b) >= 0x1p-126f && fabs(b) <= 0x1p44f)) key = 0u;
+  }
+  __device__ __forceinline__ void divisor(double b) {
+    if (!(fabs(b) >= 0x1p-1022 && fabs(b) <= 0x1p400)) key = 0u;
+  }
+  template <class T> __device__ __forceinline__ void iterate(T u) {
+    if (!(fabs(u) <= std::numeric_limits<T>::max())) key = 0u;
+  }
+  template <class T> __device__ __forceinline__ bool out() const { return key < key_of(sizeof(T) == 4 ? T(0x1p-80) : T(0x1p-600)); }
+};
+__device__ __forceinline__ float corrected(float a, float b, float y, float q) {
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
 }
-__device__ __forceinline__ double quotient(double a, double b, double y) {
-  double q = a * y;
-  q = __builtin_fma(__builtin_fma(-q, b, a), y, q);
-  q = __builtin_fma(__builtin_fma(-q, b, a), y, q);
-  return __builtin_amdgcn_div_fixup(q, b, a);
+__device__ __forceinline__ double corrected(double a, double b, double y, double q) {
+  return __builtin_fma(__builtin_fma(-q, b, a), y, q);
+}
+__device__ __forceinline__ float fixup(float q, float b, float a) { return __builtin_amdgcn_div_fixupf(q, b, a); }
+__device__ __forceinline__ double fixup(double q, double b, double a) { return __builtin_amdgcn_div_fixup(q, b, a); }
+template <class T> __device__ __forceinline__ T recip(T b, Range& off) {
+  off.divisor(b);
+  return T(1) / b;
+}
+template <class T> __device__ __forceinline__ T quotient(T a, T b, T y, Range& off) {
+  off.dividend(a);
+  T q = a * y;
+  q = corrected(a, b, y, q);
+  q = corrected(a, b, y, q);
+  return fixup(q, b, a);
 }
 
 // Offsets of the 18 neighbours of the 19-point operator in the order of its terms: faces (+-x, +-y, +-z),
@@ -115,7 +148,7 @@ template <class T, int N> struct PointOp<T, N, false> {
   int nb[18];
   T w[7], x[12], y, b, b2;
   T di2;
-  __device__ __forceinline__ void load(const T* G, const T* rhs, int p, T dx) {
+  __device__ __forceinline__ void load(const T* G, const T* rhs, int p, T dx, Range& off) {
     int i, j, k;
     point_of<1, true>(p, N, i, j, k);
 #pragma unroll
@@ -124,17 +157,17 @@ template <class T, int N> struct PointOp<T, N, false> {
     faces19<T>(w, G, N * N * N, p, nb);
 #pragma unroll
     for (int e = 0; e < 12; ++e) x[e] = G[XG19[e][1] * N * N * N + nb[XG19[e][0]]];
-    y = T(1) / w[6];
+    y = recip(w[6], off);
     b = rhs[p];
     b2 = b * (dx * dx);
     di2 = T(1) / (dx * dx);
   }
-  __device__ __forceinline__ T update(const T* u, int) const {
+  __device__ __forceinline__ T update(const T* u, Range& off) const {
     T q[18], t1, t2;
 #pragma unroll
     for (int e = 0; e < 18; ++e) q[e] = u[nb[e]];
     terms19<T>(t1, t2, w, x, q);
-    return quotient(b2 - t1 - t2, w[6], y);
+    return quotient(b2 - t1 - t2, w[6], y, off);
   }
   __device__ __forceinline__ T resid(const T* u, int p) const {
     T q[18], t1, t2;
@@ -148,7 +181,7 @@ template <class T, int N> struct PointOp<T, N, false> {
 template <class T, int N> struct PointOp<T, N, true> {
   int nb[27];
   T a[27], y, b;
-  __device__ __forceinline__ void load(const T* A, const T* rhs, int p, T) {
+  __device__ __forceinline__ void load(const T* A, const T* rhs, int p, T, Range& off) {
     int i, j, k;
     point_of<1, true>(p, N, i, j, k);
 #pragma unroll
@@ -156,7 +189,7 @@ template <class T, int N> struct PointOp<T, N, true> {
       nb[e] = (int)lx<1, true>((i + e % 3 - 1) & (N - 1), (j + e / 3 % 3 - 1) & (N - 1), (k + e / 9 - 1) & (N - 1), N);
       a[e] = A[e * N * N * N + p];
     }
-    y = T(1) / a[13];
+    y = recip(a[13], off);
     b = rhs[p];
   }
   __device__ __forceinline__ T offsum(const T* u) const {
@@ -169,7 +202,7 @@ template <class T, int N> struct PointOp<T, N, true> {
       if (e != 13) s = s + a[e] * q[e];
     return s;
   }
-  __device__ __forceinline__ T update(const T* u, int) const { return quotient(b - offsum(u), a[13], y); }
+  __device__ __forceinline__ T update(const T* u, Range& off) const { return quotient(b - offsum(u), a[13], y, off); }
   __device__ __forceinline__ T resid(const T* u, int p) const { return b - (offsum(u) + a[13] * u[p]); }
   template <class F> static __device__ __forceinline__ void phases(int ns, bool rev, F&& f) { phases27(ns, rev, f); }
 };
@@ -251,13 +284,13 @@ __device__ __forceinline__ void cc_zerosum(T* u, double* scal, int* guard, int m
 // which 64 threads hold a value, so the levels above h = 32 add zeros.
 template <class T, bool GAL>
 __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T dx, int nc, bool rev, double* scal, int* guard,
-                                          int ref, int mode) {
+                                          int ref, int mode, Range& off) {
   if (threadIdx.x >= 64) return;
   const int p = threadIdx.x;
   PointOp<T, 4, GAL> P;
-  P.load(op, rhs4, p, dx);
+  P.load(op, rhs4, p, dx, off);
   auto phase = [&](unsigned mask) {
-    if ((mask >> (p >> 3)) & 1u) u4[p] = P.update(u4, p);
+    if ((mask >> (p >> 3)) & 1u) u4[p] = P.update(u4, off);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   };
   double r1 = 0.0, re = 0.0;
@@ -265,6 +298,7 @@ __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T d
   if (ref) r1 = max64((double)fabs(P.resid(u4, p)));
   PointOp<T, 4, GAL>::phases(nc, rev, phase);
   if (ref) re = max64((double)fabs(P.resid(u4, p)));
+  off.iterate(u4[p]);
   double sum = tree64(0.0 + (double)u4[p]);
   sum = __shfl(sum, 0);
   bool g = false;
@@ -282,15 +316,16 @@ __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T d
 // maximum only.
 template <class T, bool GAL>
 __device__ __forceinline__ double cc_level8(T* u, const T* rhs, T* r8, const T* op, T dx, int ns, bool rev, int want, int norm,
-                                            Cc16Scratch& S) {
+                                            Cc16Scratch& S, Range& off) {
   const int p = threadIdx.x;
   PointOp<T, 8, GAL> P;
-  P.load(op, rhs, p, dx);
+  P.load(op, rhs, p, dx, off);
   const int cls = __builtin_amdgcn_readfirstlane(p >> 6);
   PointOp<T, 8, GAL>::phases(ns, rev, [&](unsigned mask) {
-    if ((mask >> cls) & 1u) u[p] = P.update(u, p);
+    if ((mask >> cls) & 1u) u[p] = P.update(u, off);
     __syncthreads();
   });
+  off.iterate(u[p]);
   if (!want) return 0.0;
   const T rv = P.resid(u, p);
   if (want == 1) r8[p] = rv;
@@ -335,7 +370,7 @@ template <int C = 0, class F> __device__ __forceinline__ void each_class(unsigne
 // G2, G3, G5 in LDS (big).
 template <class T>
 __device__ __forceinline__ double cc_level16_19(T* u, const T* rhs, T* r, T* big, const T* G, T dx, int ns, bool rev, int want,
-                                                int norm, Cc16Scratch& S) {
+                                                int norm, Cc16Scratch& S, Range& off) {
   constexpr bool REG = sizeof(T) == 4;
   const int q = threadIdx.x;
   Cell16 K;
@@ -359,7 +394,7 @@ __device__ __forceinline__ double cc_level16_19(T* u, const T* rhs, T* r, T* big
     faces19<T>(f, G, 4096, c * 512 + q, nb);
 #pragma unroll
     for (int e = 0; e < (REG ? 7 : 6); ++e) w[c][e] = f[e];
-    y[c] = T(1) / f[6];
+    y[c] = recip(f[6], off);
     if constexpr (REG) {
       b2[c] = rhs[c * 512 + q] * dx2;
 #pragma unroll
@@ -405,10 +440,12 @@ __device__ __forceinline__ double cc_level16_19(T* u, const T* rhs, T* r, T* big
       T t1, t2, d;
       const T b = scaled_rhs(cc);
       terms(cc, t1, t2, d);
-      u[c * 512 + q] = quotient(b - t1 - t2, d, y[c]);
+      u[c * 512 + q] = quotient(b - t1 - t2, d, y[c], off);
     });
     __syncthreads();
   });
+#pragma unroll
+  for (int c = 0; c < 8; ++c) off.iterate(u[c * 512 + q]);
   if (!want) return 0.0;
   const T di2 = T(1) / dx2;
   T rv[8];
@@ -439,7 +476,7 @@ constexpr int rank27(int e, int corner) {  // index of offset e among the corner
 }
 template <class T>
 __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big, const T* A, int ns, bool rev, int want,
-                                                int norm, Cc16Scratch& S) {
+                                                int norm, Cc16Scratch& S, Range& off) {
   constexpr bool REG = sizeof(T) == 4;
   const int q = threadIdx.x;
   Cell16 K;
@@ -456,7 +493,7 @@ __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big
         if (corner27(e)) big[rank27(e, 1) * 4096 + c * 512 + q] = v;  // read back by this thread only
         else a[c][rank27(e, 0)] = v;
       }
-      y[c] = T(1) / a[c][rank27(13, 0)];
+      y[c] = recip(a[c][rank27(13, 0)], off);
       b[c] = rhs[c * 512 + q];
     }
     auto offsum = [&](auto cc) -> T {
@@ -473,10 +510,12 @@ __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big
     phases27(ns, rev, [&](unsigned mask) {
       each_class(mask, [&](auto cc) {
         constexpr int c = decltype(cc)::value;
-        u[c * 512 + q] = quotient(b[c] - offsum(cc), a[c][rank27(13, 0)], y[c]);
+        u[c * 512 + q] = quotient(b[c] - offsum(cc), a[c][rank27(13, 0)], y[c], off);
       });
       __syncthreads();
     });
+#pragma unroll
+    for (int c = 0; c < 8; ++c) off.iterate(u[c * 512 + q]);
     if (!want) return 0.0;
     each_class(0xFFu, [&](auto cc) {
       constexpr int c = decltype(cc)::value;
@@ -561,11 +600,14 @@ template <class P> __device__ __forceinline__ P* uniform(P* p) {
   return (P*)((uint64_t)hi << 32 | lo);
 }
 
-// Levels C.n[0] (16, 8 or 4) .. 4 of the cycle C (cw_cycle's schedule), by CW threads.
-template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
+// Levels C.n[0] (16, 8 or 4) .. 4 of the cycle C (cw_cycle's schedule), by CW threads, up to the entry
+// level's iterate, which is left in LDS; whether a quotient of this thread was out of range.
+template <class T> __device__ __forceinline__ bool cc16_levels(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
   static_assert(CW == 512, "one 16^3 cell, and one 8^3 point, per thread");
   const int t = threadIdx.x, lb = C.nl - 1, l8 = C.nl - 2, l16 = C.nl - 3;
   T* r16 = M.big;
+  Range off;   // of the levels in T
+  Range offd;  // of the FP64 4^3 level (mixed)
   double r1_16 = 0.0, r1_8 = 0.0;
   // the entry level's iterate and right-hand side; coarser levels start from 0
   if (l16 >= 0) {
@@ -580,8 +622,8 @@ template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<
   }
   __syncthreads();
   if (l16 >= 0) {
-    if (C.A[l16]) r1_16 = cc_level16_27<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], false, 1, C.ref, M.S);
-    else r1_16 = cc_level16_19<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], false, 1, C.ref, M.S);
+    if (C.A[l16]) r1_16 = cc_level16_27<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], false, 1, C.ref, M.S, off);
+    else r1_16 = cc_level16_19<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], false, 1, C.ref, M.S, off);
     if (C.ref && t == 0) C.scal[l16][0] = r1_16;
     __syncthreads();
     restrict_point<T, 1, true>(M.rhs8, r16, 16, relax_plane(C.sw[l16], 16), t);
@@ -589,8 +631,8 @@ template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<
     __syncthreads();
   }
   if (l8 >= 0) {
-    if (C.A[l8]) r1_8 = cc_level8<T, true>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S);
-    else r1_8 = cc_level8<T, false>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S);
+    if (C.A[l8]) r1_8 = cc_level8<T, true>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S, off);
+    else r1_8 = cc_level8<T, false>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S, off);
     if (C.ref && t == 0) C.scal[l8][0] = r1_8;
     __syncthreads();
     if (t < 64) {
@@ -606,37 +648,62 @@ template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<
       M.du[t] = 0.0;
     }
     __syncthreads();
-    if (C.dA) cc_bottom<double, true>(M.du, M.drhs, C.dA, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b);
-    else cc_bottom<double, false>(M.du, M.drhs, C.dG, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b);
+    if (C.dA) cc_bottom<double, true>(M.du, M.drhs, C.dA, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b, offd);
+    else cc_bottom<double, false>(M.du, M.drhs, C.dG, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b, offd);
     if (t < 64) M.u4[t] = (T)M.du[t];
   } else {
-    if (C.A[lb]) cc_bottom<T, true>(M.u4, M.rhs4, C.A[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b);
-    else cc_bottom<T, false>(M.u4, M.rhs4, C.G[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b);
+    if (C.A[lb]) cc_bottom<T, true>(M.u4, M.rhs4, C.A[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b, off);
+    else cc_bottom<T, false>(M.u4, M.rhs4, C.G[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b, off);
   }
   __syncthreads();
-  if (l8 < 0) {
-    if (t < 64) C.u[lb][t] = M.u4[t];
-    return;
-  }
+  if (l8 < 0) return off.template out<T>() || offd.template out<double>();
   if (t < 64) prolong_cell<T, true>(M.u8, M.u4, 8, 1, t);
   __syncthreads();
   double re;
-  if (C.A[l8]) re = cc_level8<T, true>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
-  else re = cc_level8<T, false>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
+  if (C.A[l8]) re = cc_level8<T, true>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
+  else re = cc_level8<T, false>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
   if (C.ref && t == 0) C.scal[l8][1] = re;
   cc_zerosum<T, 8>(M.u8, C.scal[l8], C.guard[l8], (C.ref && !(C.top && l8 == 0)) ? 1 : 0, r1_8, re, M.S);
-  if (l16 < 0) {
-    C.u[l8][t] = M.u8[t];
-    return;
-  }
+  if (l16 < 0) return off.template out<T>() || offd.template out<double>();
   prolong_cell<T, true>(M.u16, M.u8, 16, 1, t);
   __syncthreads();
-  if (C.A[l16]) re = cc_level16_27<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
-  else re = cc_level16_19<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
+  if (C.A[l16]) re = cc_level16_27<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
+  else re = cc_level16_19<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
   if (C.ref && t == 0) C.scal[l16][1] = re;
   cc_zerosum<T, 16>(M.u16, C.scal[l16], C.guard[l16], (C.ref && !(C.top && l16 == 0)) ? 1 : 0, r1_16, re, M.S);
+  return off.template out<T>() || offd.template out<double>();
+}
+
+// The general form (cw_cycle), called, not inlined: its registers and the level table's indexing would
+// otherwise cost the levels on chip spills.  Scratch and the level table are in LDS.
+template <class T> struct Cc16General {
+  double s[CW / RB][RB], blk[64], blk2[64], wm[CW / 64];
+  CoarseCycle<T> C;
+};
+template <class T> __device__ __attribute__((noinline)) void cc16_general(Cc16General<T>* g) {
+  cw_cycle<T>(g->C, g->s, g->blk, g->blk2, g->wm);
+}
+
+// The cycle; off the quotients' range by the general form, from the caller's arrays, which the levels on
+// chip have only read but for the per-level scalars and guards, formed again.
+template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
+  const int t = threadIdx.x;
+  if (__syncthreads_or(cc16_levels<T>(C, M))) {
+    static_assert(sizeof(Cc16General<T>) <= sizeof(M.big), "the general form's LDS lies in the staged coefficients'");
+    Cc16General<T>* g = reinterpret_cast<Cc16General<T>*>(M.big);
+    if (t == 0) g->C = C;
+    __syncthreads();
+    cc16_general<T>(g);
+    return;
+  }
+  if (C.nl == 1) {
+    if (t < 64) C.u[0][t] = M.u4[t];
+  } else if (C.nl == 2) {
+    C.u[0][t] = M.u8[t];
+  } else {
 #pragma unroll
-  for (int c = 0; c < 8; ++c) C.u[l16][c * 512 + t] = M.u16[c * 512 + t];
+    for (int c = 0; c < 8; ++c) C.u[0][c * 512 + t] = M.u16[c * 512 + t];
+  }
 }
 
 template <class T> __global__ __launch_bounds__(CW) void k_coarse16(CoarseCycle<T> C) {
