@@ -7,7 +7,7 @@
 namespace mmh {
 
 // Position of particle p in grid units and its cell (haloden.f90:84-99): x = modulo(x, nf) * ng / nf,
-// cell = floor(x) (0-based; clamped to ng-1 where the scaled position rounds up to ng).
+// cell = floor(x) (0-based; clamped to ng-1 where the scaled position rounds up to ng, and to 0).
 __global__ void k_pd_cells(float* __restrict__ xs, int* __restrict__ cell, int* __restrict__ idx,
                            const float* __restrict__ xp, i64 np, int ng, float nf) {
   const i64 p = (i64)blockIdx.x * blockDim.x + threadIdx.x;
@@ -18,8 +18,7 @@ __global__ void k_pd_cells(float* __restrict__ xs, int* __restrict__ cell, int* 
     x = x - floorf(x / nf) * nf;  // modulo(x, real(nf))
     x = x * (float)ng / nf;
     xs[3 * p + d] = x;
-    int ci = (int)floorf(x);
-    c[d] = ci < 0 ? 0 : (ci > ng - 1 ? ng - 1 : ci);
+    c[d] = x >= 1.f ? (x < (float)ng ? (int)x : ng - 1) : 0;  // NaN: 0
   }
   cell[p] = c[0] + ng * (c[1] + ng * c[2]);
   idx[p] = (int)p;
@@ -109,7 +108,7 @@ struct PdSearch {
   int ng, rmax;
 };
 
-// The empty cell c's particle, searched from half-width r0 on (FIRST: only r = 1; -1 if its cube is empty).
+// The empty cell c's particle, searched from half-width r0 on (FIRST: only r = 1; -1 if its cube holds none).
 template <bool FIRST> __device__ __forceinline__ int pd_search(const PdSearch& P, unsigned c, int r0) {
   const int ng = P.ng, rw = pd_row_words(ng);
   const unsigned row = c / (unsigned)ng;
@@ -185,7 +184,7 @@ template <bool FIRST> __device__ __forceinline__ int pd_search(const PdSearch& P
 }
 
 // First pass over all cells, PD_CH x 256 of them per workgroup at most: -1 for the non-empty ones, the
-// cells whose cube r = 1 holds a particle, and the others into far (their count in far[0]) for a second
+// cells that find theirs in the cube r = 1, and the others into far (their count in far[0]) for a second
 // pass, where the wider searches fill whole wavefronts instead of a few lanes of each.  The list is
 // gathered in LDS and takes one atomic of the workgroup: an atomic per wavefront on the one counter
 // cost 1.2 ms at 200^3.
@@ -209,7 +208,10 @@ __global__ __launch_bounds__(256) void k_pd_nearest(int* __restrict__ near, int*
       const int x0 = (int)(c - row * P.ng) - 1 + 32;
       const unsigned* w = P.near + (int)row * rw + (x0 >> 5);
       wide = !((unsigned)((((uint64_t)w[1] << 32) | w[0]) >> ((unsigned)x0 & 31u)) & 7u);
-      if (!wide) best = pd_search<true>(P, c, 1);
+      if (!wide) {
+        best = pd_search<true>(P, c, 1);
+        wide = best < 0;  // only particles without a distance (NaN coordinates) in the cube
+      }
     }
     if (c < ncell) near[c] = best;
     if (wide) list[atomicAdd(&count, 1)] = (int)c;

@@ -28,3 +28,26 @@ def test_search_matches_oracle(ctx, ng, npart, clump):
         ctx.particle_density(torch.from_numpy(xp).cuda(), ng, 2.0 * ng, den, wp)
         assert np.array_equal(wp.cpu().numpy(), wp_o)
         assert np.allclose(den.cpu().numpy(), den_o.ravel(), rtol=1.2e-7, atol=0)
+
+
+@pytest.mark.parametrize("ng,npart", [(6, 3), (20, 60), (33, 900)])
+def test_particles_without_a_position_attract_no_cell(ctx, ng, npart):
+    """A particle of NaN coordinates lies in the first cell and is at no distance from any other: the empty
+    cells around it find theirs in wider cubes, as without it."""
+    print("case particle search with NaN ng=%d np=%d" % (ng, npart), flush=True)
+    rng = np.random.default_rng(ng)
+    x = (1.0 + rng.random((npart, 3)) * (ng - 1)).astype(np.float32)  # none in the first cell's planes
+    _, wp_o = R.or_particle_density(x, ng, float(ng))
+    # the first cell's own particle without the NaN one: nearest in the smallest cube that holds any
+    cell = np.floor(x).astype(int)
+    d = np.minimum(np.abs(x - np.float32(0.5)), ng - np.abs(x - np.float32(0.5)))
+    cube = np.minimum(cell, ng - cell).max(1)
+    first = cube == cube.min()
+    p0 = np.flatnonzero(first)[np.argmin((d[first].astype(np.float64) ** 2).sum(1))]
+    wp_o = wp_o.copy()
+    wp_o[p0] -= 1
+    xn = np.concatenate([x, np.full((1, 3), np.nan, np.float32)])
+    den = torch.zeros(ng ** 3, dtype=torch.float32, device="cuda")
+    wp = torch.zeros(npart + 1, dtype=torch.int32, device="cuda")
+    ctx.particle_density(torch.from_numpy(xn).cuda(), ng, float(ng), den, wp)
+    assert np.array_equal(wp.cpu().numpy(), np.append(wp_o, 1))
