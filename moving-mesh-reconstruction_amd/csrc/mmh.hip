@@ -2568,16 +2568,18 @@ int mmh_particle_density_f(mmh_ctx* c, const float* xp, long long np, int ng, fl
     float4* xo = (float4*)ws_get(c, "pd_xo", sizeof(float4) * np);
     const i64 nwords = (i64)pd_row_words(ng) * ng * ng;
     unsigned* occ = (unsigned*)ws_get(c, "pd_occ", sizeof(unsigned) * (1 + PD_NEAR) * nwords);
-    k_pd_sorted<<<nblk(np), 256, 0, c->stream>>>(xo, order, xs, np);
+    int* far = (int*)ws_get(c, "pd_far", sizeof(int) * (2 + ncell));  // out flag, then the far list behind its count
+    k_fill<int><<<1, 64, 0, c->stream>>>(far, 0, 2);
+    int* out = far++;
+    k_pd_sorted<<<nblk(np), 256, 0, c->stream>>>(xo, out, order, xs, np, (float)ng);
     k_pd_bits<<<nblk(32 * nwords), 256, 0, c->stream>>>(occ, start, end, ng, nwords);
     k_pd_bits_near<<<nblk(nwords), 256, 0, c->stream>>>(occ + nwords, occ, ng, nwords);
-    int* far = (int*)ws_get(c, "pd_far", sizeof(int) * (1 + ncell));
-    k_fill<int><<<1, 64, 0, c->stream>>>(far, 0, 1);
-    const PdSearch P{start, end, xo, occ, occ + nwords, nwords, ng, ng / 2 + 1};
+    const PdSearch P{start, end, xo, occ, occ + nwords, out, nwords, ng, ng / 2 + 1};
     // enough workgroups for the chip first, then longer ones
     const int chunks = (int)std::min<i64>(PD_CH, std::max<i64>(1, ncell / 256 / 2048));
     k_pd_nearest<<<nblk(ncell, 256 * chunks), 256, 0, c->stream>>>(near, wp, far, P, chunks);
     k_pd_far<<<(unsigned)std::min<i64>(nblk(ncell), 8192), 256, 0, c->stream>>>(near, wp, far, P);
+    k_pd_out<<<(unsigned)std::min<i64>(nblk(ncell), 512), 256, 0, c->stream>>>(near, wp, P);
     k_pd_density<<<nblk(ncell), 256, 0, c->stream>>>(den, near, wp, start, end, order, ncell);
     LAUNCHCHK();
     double* sum = wsT<double>(c, "pd_sum", 1);

@@ -51,3 +51,22 @@ def test_particles_without_a_position_attract_no_cell(ctx, ng, npart):
     wp = torch.zeros(npart + 1, dtype=torch.int32, device="cuda")
     ctx.particle_density(torch.from_numpy(xn).cuda(), ng, float(ng), den, wp)
     assert np.array_equal(wp.cpu().numpy(), np.append(wp_o, 1))
+
+
+@pytest.mark.parametrize("ng,npart,boxes", [(12, 40, 2.0 ** 26), (33, 500, 2.0 ** 25), (33, 500, 2.0 ** 20)])
+def test_coordinates_far_outside_the_box(ctx, ng, npart, boxes):
+    """Coordinates millions of boxes out, whose modulo in FP32 leaves the box: distances to them are periodic
+    all the same.  Counts match exactly."""
+    print("case particle search far ng=%d boxes=%g" % (ng, boxes), flush=True)
+    rng = np.random.default_rng(ng)
+    nf = np.float32(3.7)
+    x = rng.random((npart, 3)) * nf
+    far = rng.random((npart, 3)) < 0.3
+    x[far] += nf * np.round(boxes * rng.standard_normal(int(far.sum())))
+    xp = x.astype(np.float32)
+    den_o, wp_o = R.or_particle_density(xp, ng, float(nf))
+    den = torch.zeros(ng ** 3, dtype=torch.float32, device="cuda")
+    wp = torch.zeros(npart, dtype=torch.int32, device="cuda")
+    ctx.particle_density(torch.from_numpy(xp).cuda(), ng, float(nf), den, wp)
+    assert np.array_equal(wp.cpu().numpy(), wp_o)
+    assert np.allclose(den.cpu().numpy(), den_o.ravel(), rtol=1.2e-7, atol=0)
