@@ -88,9 +88,10 @@ __global__ void k_mismatch(T* __restrict__ tmp, T* __restrict__ rho, const T* __
 }
 
 // Diagnostics of a workgroup: thread values combined over the wavefront and then the workgroup, stored
-// at part[f gridDim.x + block].  Maxima, minima and counts do not depend on the order.
+// at part[f gridDim.x + block].  Maxima, minima and counts do not depend on the order: a value that is
+// NaN is passed over (a, the value so far, never is one).
 template <int OP> __device__ __forceinline__ double stat_op(double a, double b) {
-  return OP == 0 ? a + b : (OP == 1 ? dmax(a, b) : dmin(a, b));
+  return OP == 0 ? a + b : (OP == 1 ? (b > a ? b : a) : (b < a ? b : a));
 }
 template <int OP> __device__ __forceinline__ void block_stat(double a, double* part, int f) {
   __shared__ double w[4];
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(256) void k_stats(double* __restrict__ out, const d
     if (op == 0 && b < nb) a = part[f * nb + b];
     for (b += (i64)gridDim.x * 256; b < nb; b += (i64)gridDim.x * 256) {
       const double v = part[f * nb + b];
-      a = op == 0 ? a + v : (op == 1 ? dmax(a, v) : dmin(a, v));
+      a = op == 0 ? stat_op<0>(a, v) : (op == 1 ? stat_op<1>(a, v) : stat_op<2>(a, v));
     }
     if (op == 0) block_stat<0>(a, out, f);
     else if (op == 1) block_stat<1>(a, out, f);
@@ -160,8 +161,8 @@ __global__ __launch_bounds__(256) void k_lim_point(T* __restrict__ s, unsigned c
     const bool ex = det > T(10.0f);
     P.put(flag, (unsigned char)((ex ? 1 : 0) | (tlim > T(0) ? 2 : 0)));
     nexp += ex ? 1.0 : 0.0;
-    dhi = dmax(dhi, (double)det);
-    dlo = dmin(dlo, (double)det);
+    dhi = stat_op<1>(dhi, (double)det);
+    dlo = stat_op<2>(dlo, (double)det);
   }
   block_stat<0>(nexp, part, 0);
   block_stat<1>(dhi, part, 1);
@@ -202,8 +203,8 @@ __global__ __launch_bounds__(256) void k_eflux(T* __restrict__ eflux, const T* _
     ef = dmax(-T(1.) / dtaumesh, ef);
     P.put(eflux, ef);
     if (gate) P.put(gate, dm);
-    fhi = dmax(fhi, (double)(ef * dtold));
-    flo = dmin(flo, (double)(ef * dtold));
+    fhi = stat_op<1>(fhi, (double)(ef * dtold));
+    flo = stat_op<2>(flo, (double)(ef * dtold));
   }
   block_stat<1>(fhi, part, 0);
   block_stat<2>(flo, part, 1);
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(256) void k_complim(T* __restrict__ lim, const T* _
     T v = T(0.);
     if (tlim > T(0)) { v = tlim; c0 += 1.0; }
     P.put(lim, v);
-    c1 = dmax(c1, (double)compression);
+    c1 = stat_op<1>(c1, (double)compression);
   }
   block_stat<0>(c0, part, 0);
   block_stat<1>(c1, part, 1);

@@ -44,3 +44,22 @@ def test_limiter_diagnostics(ctx, n):
     for f in ("detmin", "detmax", "fluxmin", "fluxmax"):
         assert getattr(st, f) == getattr(st_o, f), f
     assert abs(st.cmax - st_o.cmax) <= 1e-12 * abs(st_o.cmax)  # device acos and cos
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("n,k", [(16, 0), (16, 1), (64, 33)])
+def test_limiter_extremes_beside_a_nan(ctx, n, k, dt):
+    """A mesh potential that is NaN at one point: the determinant's extremes are those of the other points (of
+    a spike two planes away and its mirror images, which the NaN does not reach)."""
+    print("case limiter NaN n=%d k=%d %s" % (n, k, dt.__name__), flush=True)
+    d = np.zeros((n, n, n), dt)  # [k, j, i]
+    d[k, 7, 7] = -1.0            # det = 27 at the spike, and 0 or below around it
+    u = np.zeros((n ** 3, 5), dt)
+    u[:, 0] = 1.0
+    new = lambda m=n ** 3: np.zeros(m, dt)  # noqa: E731
+    ref = R.or_calcdefp(new(), new(), new((n + 2) * n * n), d.ravel(), u.ravel(), n, sumorder=2)
+    d[k + 2, 7, 7] = np.nan
+    to = lambda a: torch.from_numpy(a.ravel()).cuda()  # noqa: E731
+    st = ctx.calcdefp(to(new()), to(new()), to(new((n + 2) * n * n)), to(d), to(u))
+    assert ref.detmax == 27.0
+    assert (st.detmax, st.detmin) == (ref.detmax, ref.detmin)
