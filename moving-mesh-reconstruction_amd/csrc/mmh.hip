@@ -1045,6 +1045,9 @@ template <class T> const T* cosine_table(mmh_ctx* c, int n) {
   return cs;
 }
 
+// Side of the largest fields the pointwise and spectral calls take (n^3 work-items make one launch).
+constexpr int FIELD_N = 1024;
+
 // out = inverse transform of the multiplier `mode` times the spectrum whose forward complex
 // transform (three axes, not yet recombined) is `spec` (may equal out): the middle of the operation
 // and the inverse x lines in one pass, then the y and z axes.  speq (may be null): the Nyquist
@@ -1059,8 +1062,8 @@ void spectral_inverse(mmh_ctx* c, T* out, const T* spec, T* speq, int n, int mod
   C2<T>* z = reinterpret_cast<C2<T>*>(out);
   const i64 total = cube(n) / 2;
   for_line(n / 2, [&](auto len) {
-    constexpr int L = std::min(decltype(len)::value, 1024), NP = 128 / FftShape<L>::TL;
-    require(2 * L == n, "spectral: n up to 2048");
+    constexpr int L = std::min(decltype(len)::value, FIELD_N / 2), NP = 128 / FftShape<L>::TL;
+    require(2 * L == n, "spectral: n up to 1024");
     const i64 pairs = (i64)(L - 1) * n + 2 * (L + 1);
     k_rlft_mid<T, L><<<(unsigned)((pairs + NP - 1) / NP), 256, 0, c->stream>>>(
         z, reinterpret_cast<const C2<T>*>(spec), Wp, Wm, W, reinterpret_cast<C2<T>*>(speq), mode, zero_dc, cs, piG);
@@ -1079,6 +1082,7 @@ template <class T> void smooth(mmh_ctx* c, T* out, const T* in, int n) {
 }
 // nsmooth of a, `times` over.
 template <class T> void nsmooth_dev(mmh_ctx* c, T* a, int n, int times) {
+  require(n <= FIELD_N, "nsmooth: n up to 1024");
   T* t = wsT<T>(c, "smooth_tmp", cube(n));
   for (; times >= 2; times -= 2) {
     smooth(c, t, a, n);
@@ -1288,6 +1292,7 @@ void reconstruct_dev(mmh_ctx* c, T* u, T* def, T* defp, int n, int nf, int niter
 }
 
 template <class T> void spectral_out(mmh_ctx* c, const T* phi, T* out, int n, int mode) {
+  require(n <= FIELD_N, "spectral: n up to 1024");
   T* d = wsT<T>(c, "specD", cube(n));
   fft3_dev<T>(c, reinterpret_cast<C2<T>*>(d), reinterpret_cast<const C2<T>*>(phi), n / 2, n, n, 1);
   spectral_inverse<T>(c, out, d, nullptr, n, mode, 0, T(1) / T(n));
@@ -1295,6 +1300,7 @@ template <class T> void spectral_out(mmh_ctx* c, const T* phi, T* out, int n, in
 
 // scalar2gradient: the three components from one forward transform.
 template <class T> void gradient_dev(mmh_ctx* c, const T* phi, T* psi, int n) {
+  require(n <= FIELD_N, "gradient: n up to 1024");
   T* d = wsT<T>(c, "specD", cube(n));
   fft3_dev<T>(c, reinterpret_cast<C2<T>*>(d), reinterpret_cast<const C2<T>*>(phi), n / 2, n, n, 1);
   for (int a = 0; a < 3; ++a) spectral_inverse<T>(c, psi + (i64)a * cube(n), d, nullptr, n, 2 + a, 0, T(1) / T(n));

@@ -70,3 +70,11 @@ def test_coordinates_far_outside_the_box(ctx, ng, npart, boxes):
     ctx.particle_density(torch.from_numpy(xp).cuda(), ng, float(nf), den, wp)
     assert np.array_equal(wp.cpu().numpy(), wp_o)
     assert np.allclose(den.cpu().numpy(), den_o.ravel(), rtol=1.2e-7, atol=0)
+
+
+@pytest.mark.parametrize("ng,npart,clump", [(103, 20001, 1), (103, 3000, 0), (130, 300000, 0), (207, 400000, 0)])
+def test_workgroups_of_several_chunks(ctx, ng, npart, clump):
+    """Grids whose workgroups of the first pass take 2, 4 and 16 chunks of cells (from 2^20 cells on), the last
+    of them past the end, with a few cells for the second pass and with most.  As above."""
+    print("case particle chunks ng=%d np=%d" % (ng, npart), flush=True)
+    test_search_matches_oracle(ctx, ng, npart, clump)

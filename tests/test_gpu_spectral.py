@@ -47,3 +47,16 @@ def test_rlft3_both_ways_equals_the_oracle(ctx, n):
         R.or_rlft3(a, sq, n, sign)
         ctx.rlft3(ad, sd, sign)
         assert np.array_equal(ad.cpu().numpy(), a) and np.array_equal(sd.cpu().numpy(), sq)
+
+
+def test_fields_of_more_than_a_launch_are_refused(ctx):
+    """2048^3 points: refused, and the field is left as it was."""
+    import mmh_amd
+    print("case spectral n=2048 refused", flush=True)
+    a = torch.zeros(2048 ** 3, dtype=torch.float32, device="cuda")
+    a[12345] = 1.0
+    for call in (lambda: ctx.defp2delta(a, a), lambda: ctx.nsmooth(a)):
+        with pytest.raises(mmh_amd.MmhError) as e:
+            call()
+        assert e.value.code == mmh_amd.MMH_EINVAL
+    assert float(a[12345]) == 1.0 and int(torch.count_nonzero(a[:1 << 20])) == 1
