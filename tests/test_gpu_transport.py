@@ -1,6 +1,6 @@
 """GPU: the transport step against the oracle on a fluid with momentum and energy, at every tile
-shape of the march (16 and 32 wide, 64 wide) and walk length.  Halvings taken together are exact, so
-the bar is equality."""
+shape of the march (16, 32 and 64 wide) and both walk lengths that occur: 4 planes up to 128^3, 32
+from 256^3.  Halvings taken together are exact, so the bar is equality."""
 import numpy as np
 import pytest
 
@@ -35,3 +35,9 @@ def test_transport_of_a_flow_equals_the_oracle(ctx, n, dt):
     ctx.relaxing(got, torch.from_numpy(d).cuda(), torch.from_numpy(p).cuda(), dt=0.7)
     R.or_relaxing(u, d, p, n, dt=0.7)
     assert np.array_equal(got.cpu().numpy(), u)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_transport_by_long_walks_equals_the_oracle(ctx, dt):
+    """256^3, where a workgroup walks 32 planes."""
+    test_transport_of_a_flow_equals_the_oracle(ctx, 256, dt)
