@@ -133,6 +133,8 @@ int mmh_release_workspace(mmh_ctx* ctx);            /* free cached device buffer
  *                 the residual recurrence and the stopping test stay FP64
  *   "coarse_lds"  1 (default) / 0: the one-workgroup cycle holds its levels on chip while it runs
  *                 (16^3 and below: iterate in LDS, coefficients in registers; bit-identical)
+ *   "colour_fused" 1 (default) / 0: sweeps of small levels (64^3 and 32^3 Galerkin levels, 19-point levels
+ *                 below 256^3) update two or all eight colours in one launch, or one (bit-identical)
  *   "sweep_slabs" 4 (default), 2, 8, 16, 32 or 0: the mixed solve's finest-level sweeps (n >= 512)
  *                 run all colours on one k-slab before the next (this many slabs; the reverse
  *                 sweep in exactly reverse order).  Another Gauss-Seidel order: the preconditioner

@@ -72,7 +72,7 @@ void batch_sweeps(mmh_ctx* c, BatchGroup& g, double* phi, const double* rhs, con
   const double dx2 = g.dx[l] * g.dx[l];
   const int bsz = shape.first;
   const unsigned nb = nblk(h3, bsz);
-  colour_steps(ns, reverse, true, from_zero, [&](int col, bool pair, bool first, unsigned done) {
+  colour_steps(ns, reverse, c->colour_fused, from_zero, [&](int col, bool pair, bool first, unsigned done) {
     const dim3 grid(pair ? 2 * nb : nb, g.B);
     if (first && from_zero)
       k_colour<double, 1, false, true><<<grid, bsz, 0, c->stream>>>(phi, rhs, G, m, dx2, col >> 2, (col >> 1) & 1, col & 1,

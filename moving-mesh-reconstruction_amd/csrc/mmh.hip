@@ -61,6 +61,7 @@ struct mmh_ctx {
   int coarse_fused_ref = 16;  // the reference V-cycle's levels <= this size in one workgroup (option "coarse_fused_ref")
   int zero_start = 1;      // first sweep from u = 0 reads only the colour classes already updated (option "zero_start")
   int colour_col = 8;      // colour kernels of levels n >= colour_col_min_n: points per thread along k (option "colour_col": 1 .. 16)
+  int colour_fused = 1;    // small levels: several colours of a sweep in one launch (option "colour_fused")
   int colour_col_min_n = 256;  // below 256^3 the n^3/(8S) threads are too few to fill the GPU
   int pcg_graph = 1;       // single solve: replay the PCG preconditioner as a captured HIP graph
   int batch_graph = 1;     // batched solve: replay one PCG iteration as a captured HIP graph
@@ -634,7 +635,7 @@ void sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* G, int n, T dx, int ns, 
     ns -= 2 * pairs;
   }
   const int S = (layout == 1 && n >= c->colour_col_min_n && h % c->colour_col == 0) ? c->colour_col : 1;
-  if (layout == 1 && !delta && S == 1 && n == TILE_N) {
+  if (c->colour_fused && layout == 1 && !delta && S == 1 && n == TILE_N) {
     tile_sweeps<false, T, TG>(c, phi, rhs, G, n, dx2, ns, reverse);
     return;
   }
@@ -678,7 +679,7 @@ void sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* G, int n, T dx, int ns, 
   }
   // paired colours on the levels of one thread per point, which the launches bound: per sweep 64^3 FP32 25.4 ->
   // 19.7 us, FP64 30.4 -> 23.3 us; 128^3 40.3 -> 36.8, 64.7 -> 59.7 us
-  colour_steps(ns, reverse, layout == 1 && S == 1 && !delta, from_zero, [&](int col, bool pair, bool first, unsigned done) {
+  colour_steps(ns, reverse, c->colour_fused && layout == 1 && S == 1 && !delta, from_zero, [&](int col, bool pair, bool first, unsigned done) {
     const int kp = col >> 2, io = (col >> 1) & 1, jo = col & 1;
     const unsigned nbp = pair ? 2 * nb : nb;
     if (S > 1) colour_col_launch<T, TG>(c, S, first && from_zero, delta, phi, rhs, G, n, dx2, kp, io, jo, done);
@@ -715,11 +716,11 @@ void relax_dev(mmh_ctx* c, T* phi, const T* rhs, const TG* G, T* rscratch, int n
 // residual stored in r and restricted into rc with calcresid's plane order rule.
 template <class T, class TG = T>
 void gal_sweeps(mmh_ctx* c, T* phi, const T* rhs, const TG* A, int n, int ns, bool reverse, bool from_zero = false) {
-  if (n == TILE_N) {
+  if (c->colour_fused && n == TILE_N) {
     tile_sweeps<true, T, TG>(c, phi, rhs, A, n, T(0), ns, reverse);
     return;
   }
-  if (n == GAL_PAIR_N) {
+  if (c->colour_fused && n == GAL_PAIR_N) {
     // colours two by two (k_gal_pair)
     constexpr unsigned nbp = GAL_PAIR_N / 2 * GAL_PAIR_N / 2 / GAL_PAIR_W, nt = GAL_PAIR_N / 2 * GAL_PAIR_W;
     for (int s = 0; s < ns; ++s)
@@ -2319,6 +2320,8 @@ int mmh_set_option(mmh_ctx* c, const char* key, int value) {
       c->sweep_slabs = value;
     } else if (k == "coarse_lds") {
       c->coarse_lds = value ? 1 : 0;
+    } else if (k == "colour_fused") {
+      c->colour_fused = value ? 1 : 0;
     } else if (k == "dots32") {
       c->dots32 = value ? 1 : 0;
     } else if (k == "batch_coarse_fused") {
@@ -2360,7 +2363,7 @@ int mmh_get_option(mmh_ctx* c, const char* key, int* value) {
         {"mesh_tol", c->mesh_tol}, {"mesh_cycles", c->mesh_cycles}, {"precond_bf16", c->precond_bf16},
         {"batch_persistent", c->batch_persistent}, {"batch_coarse_fused", c->batch_coarse_fused},
         {"coarse_lds", c->coarse_lds}, {"sweep_slabs", c->sweep_slabs},
-        {"dots32", c->dots32}};
+        {"dots32", c->dots32}, {"colour_fused", c->colour_fused}};
     auto it = v.find(k);
     if (it == v.end()) throw MmhError(MMH_EINVAL, std::string("get_option: unknown key ") + key);
     *value = it->second;

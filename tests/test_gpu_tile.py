@@ -116,3 +116,36 @@ def test_galerkin_tile_sweeps_inside_a_solve(ctx, mixed, nu):
     r = torch.zeros_like(b)
     ctx.residual(r, phi, b, d, ud)
     assert float(r.abs().max()) <= 1.01e-9 * float(b.abs().max())
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+@pytest.mark.parametrize("n,galerkin,nu", [(32, 0, 2), (64, 1, 1), (64, 1, 2), (64, 1, 3), (64, 0, 2), (128, 1, 1),
+                                           (128, 1, 2), (128, 1, 3)])
+def test_colours_in_one_launch_or_eight(ctx, n, galerkin, nu, mixed):
+    """Krylov solves whose 32^3 and 64^3 levels (19-point or Galerkin, bfloat16 coefficients when mixed; from zero
+    and from a value, forward and reversed) are swept with several colours a launch, against one
+    colour a launch (option colour_fused 0): the same residual after every iteration, the same solution."""
+    print("case colours n=%d galerkin=%d nu=%d mixed=%d" % (n, galerkin, nu, mixed), flush=True)
+    rng = np.random.default_rng(nu)
+    u = np.zeros((n ** 3, 5))
+    u[:, 0] = R.or_lognormal(n, 1.5, 3)
+    d = rng.standard_normal(n ** 3)
+    for _ in range(6):
+        R.or_nsmooth(d, n)
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a).ravel()).cuda()  # noqa: E731
+    rhs, ud, d = rng.standard_normal(n ** 3), to(u), to(d)
+    out = []
+    for fused in (1, 0):
+        ctx.set_option("colour_fused", fused)
+        ctx.set_option("galerkin", galerkin)
+        try:
+            phi = to(np.zeros(n ** 3))
+            st, ok = ctx.solve(phi, to(rhs), d, ud, tol=1e-9, max_cycles=200, schedule=1, nu_pre=nu, nu_post=nu,
+                               nu_coarse=4, mixed=mixed, nu=5, krylov=True)
+        finally:
+            ctx.set_option("colour_fused", 1)
+            ctx.set_option("galerkin", 1)
+        assert ok
+        out.append((phi.cpu().numpy(), [st.relres[i] for i in range(st.cycles)]))
+    assert len(out[0][1]) > 3 and out[0][1] == out[1][1]
+    assert np.array_equal(out[0][0], out[1][0])
