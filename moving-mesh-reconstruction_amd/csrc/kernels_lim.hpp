@@ -364,7 +364,9 @@ __global__ __launch_bounds__(256) void k_tvd_flux(T* __restrict__ V, T* __restri
 // 1.5, wbee = 1 (mmh/relaxgl.f90:8): (sign a + sign b) m / 2 with m = min(1.5 x, y + 0 x), x and y
 // the smaller and larger of |a|, |b|.  The sign factor is chosen from the sign bits (0 or +-1/2) and the
 // multiply-adds are explicit where the product is exact, so this rounds, and passes on
-// infinities and NaN, as the plain expression does.
+// infinities and NaN, as the plain expression does.  Halvings are exact on normal numbers: below 2^-125 in
+// FP32 (2^-1021) the plain form rounds halves that this form keeps, by a subnormal step at most, and
+// doubled values overflow one binade sooner.
 __device__ __forceinline__ float half_sign(float a, float b) {
   const int sa = __float_as_int(a), sb = __float_as_int(b);
   return (sa ^ sb) < 0 ? 0.f : __int_as_float((sa & (int)0x80000000) | 0x3f000000);

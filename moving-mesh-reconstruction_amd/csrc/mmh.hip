@@ -459,7 +459,10 @@ unsigned march_op(mmh_ctx* c, T* out, double* bres, const T* phi, const T* rhs, 
 }
 
 // Levels whose residual is formed a thread per point (k_resid_pt): those the k-marching kernel does not take
-// (n < 64), and 64^3 by itself or in pairs.  128^3 is faster marched (31 against 50 us in FP64).
+// (n < 64), at any stack size (FP64 against the cell form: 32^3 grids, 1: 5.0 / 16.9 us, 13: 13.9 / 22.4, 48:
+// 38.2 / 41.0, 100: 74 / 85, 300: 253 / 274; 16^3, 24: 6.6 / 19.6, 300: 31 / 39), and 64^3 up to two grids
+// (1: 9.4 / 16.2 us marched, 2: 15.3 / 17.0; three would take about 21 against 17.9).  128^3 is faster
+// marched (31 against 50 us in FP64).
 inline bool resid_pt(int n, int B) { return n < 64 || (n == 64 && B <= 2); }
 // Block results of op_resid at most, per grid.
 inline unsigned resid_blocks(int n) { return n <= 64 ? nblk(cube(n), RB) : stencil_grid(n, 1); }
@@ -505,8 +508,6 @@ template <class T> void relayout(mmh_ctx* c, T* dst, const T* src, int n, int co
   LAUNCHCHK();
 }
 
-// ns colour sweeps of phi: 8 launches per sweep, one per colour class; layout 1 (sub-lattice, the
-// V-cycle's) or 0 (column-major).
 // Tile shape of the wavefront sweep: FP32 64 x 32, FP64 32 x 32 points (four LDS planes stay
 // under 64 KiB, two workgroups per CU).
 template <class T> struct WaveTile;
@@ -614,6 +615,9 @@ static int half_slab_per(int n) {
   return std::max(1, (511 + nb) / nb);
 }
 
+// ns colour sweeps of phi; layout 1 (sub-lattice, the V-cycle's) or 0 (column-major: 8 launches per sweep).
+// In layout 1 the 19-point levels take, by size, one launch per sweep (32^3), 6 (paired colours, below
+// colour_col_min_n), 8 by columns, or 8 per slab of planes (slab_now; FP32 from HALF_SLAB_MIN_N).
 // from_zero: phi is 0 on entry, so the first sweep's colours read only the classes updated before
 // them in that sweep (k_colour's MASK form; same values).
 template <class T, class TG = T>
