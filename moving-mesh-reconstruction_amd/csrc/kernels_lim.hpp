@@ -268,34 +268,18 @@ template <class T> __global__ void k_add(T* __restrict__ y, const T* __restrict_
 // caller's u(5, ...), copied into U, and the freezing speed c (cflkeuler, 1067-1139) is formed and
 // stored; otherwise the fluid is U and c is read.  n is a power of two, n^2 a multiple of 256, so a
 // workgroup's points lie in one plane: plane bases are scalars and a lane adds its offset in the plane.
-// 512^3 FP32: 3.74 ms first, 2.73 ms second (4.0-4.5 TB/s); 256^3 FP64: 0.89, 0.71 ms.
+// 512^3 FP32: 3.77 ms first, 2.70 ms second (4.0-4.5 TB/s); 256^3 FP64: 0.89, 0.71 ms.
 template <class T, bool FIRST>
 __global__ __launch_bounds__(256) void k_tvd_flux(T* __restrict__ V, T* __restrict__ U, T* __restrict__ c,
                                                   const T* __restrict__ u, const T* __restrict__ def,
                                                   const T* __restrict__ defp, int n) {
-  const int lg = __builtin_ctz(n), m = n - 1;
-  const i64 n3 = (i64)1 << (3 * lg);
-  const i64 p0 = (i64)blockIdx.x * 256;
-  const int k = (int)(p0 >> (2 * lg));
-  const int r = (int)(p0 - ((i64)k << (2 * lg))) + (int)threadIdx.x;
-  const int i = r & m, j = r >> lg;
-  const int is[3] = {(i - 1) & m, i, (i + 1) & m}, js[3] = {((j - 1) & m) << lg, j << lg, ((j + 1) & m) << lg};
-  auto at = [&](const T* f, int di, int dj, int dk) -> T {
-    return *(const T*)((const char*)(f + ((i64)((k + dk) & m) << (2 * lg))) +
-                       (uint32_t)(is[di + 1] + js[dj + 1]) * (uint32_t)sizeof(T));
-  };
-  const i64 pl = (i64)k << (2 * lg);
-  const uint32_t o = (uint32_t)r * (uint32_t)sizeof(T);
-  auto st = [&](T* f, T v) { *(T*)((char*)(f + pl) + o) = v; };
-  // H = Hess(def) as hess() forms it; b = adj(A) / det, A = I + H (882-901)
-  const T f0 = at(def, 0, 0, 0);
-  const T hxx = (at(def, 1, 0, 0) - T(2) * f0 + at(def, -1, 0, 0));
-  const T hyy = (at(def, 0, 1, 0) - T(2) * f0 + at(def, 0, -1, 0));
-  const T hzz = (at(def, 0, 0, 1) - T(2) * f0 + at(def, 0, 0, -1));
-  const T a12 = (at(def, 1, 1, 0) - at(def, -1, 1, 0) - at(def, 1, -1, 0) + at(def, -1, -1, 0)) / T(4);
-  const T a23 = (at(def, 0, 1, 1) - at(def, 0, 1, -1) - at(def, 0, -1, 1) + at(def, 0, -1, -1)) / T(4);
-  const T a13 = (at(def, 1, 0, 1) - at(def, -1, 0, 1) - at(def, 1, 0, -1) + at(def, -1, 0, -1)) / T(4);
-  const T a11 = T(1) + hxx, a22 = T(1) + hyy, a33 = T(1) + hzz;
+  const PlanePoint P(n, blockIdx.x);
+  const i64 n3 = (i64)1 << (3 * P.lg), pl = P.pl;
+  const uint32_t o = P.r * (uint32_t)sizeof(T);
+  // b = adj(A) / det, A = I + H (882-901)
+  const Hs<T> h = hess(def, P);
+  const T a12 = h.xy, a23 = h.yz, a13 = h.xz;
+  const T a11 = T(1) + h.xx, a22 = T(1) + h.yy, a33 = T(1) + h.zz;
   const T rg = a11 * a22 * a33 + T(2) * a12 * a13 * a23 - (a13 * a13) * a22 - a11 * (a23 * a23) - (a12 * a12) * a33;
   const T B1 = (a22 * a33 - a23 * a23) / rg;
   const T B2 = (a13 * a23 - a12 * a33) / rg;
@@ -303,9 +287,9 @@ __global__ __launch_bounds__(256) void k_tvd_flux(T* __restrict__ V, T* __restri
   const T B4 = (a11 * a33 - a13 * a13) / rg;
   const T B5 = (a12 * a13 - a11 * a23) / rg;
   const T B6 = (a11 * a22 - a12 * a12) / rg;
-  const T pdx = (at(defp, 1, 0, 0) - at(defp, -1, 0, 0)) / T(2);
-  const T pdy = (at(defp, 0, 1, 0) - at(defp, 0, -1, 0)) / T(2);
-  const T pdz = (at(defp, 0, 0, 1) - at(defp, 0, 0, -1)) / T(2);
+  const T pdx = (P.at(defp, 1, 0, 0) - P.at(defp, -1, 0, 0)) / T(2);
+  const T pdy = (P.at(defp, 0, 1, 0) - P.at(defp, 0, -1, 0)) / T(2);
+  const T pdz = (P.at(defp, 0, 0, 1) - P.at(defp, 0, 0, -1)) / T(2);
   T ul[5];
 #pragma unroll
   for (int l = 0; l < 5; ++l) {
@@ -316,7 +300,7 @@ __global__ __launch_bounds__(256) void k_tvd_flux(T* __restrict__ V, T* __restri
   T cp;
   if constexpr (FIRST) {
 #pragma unroll
-    for (int l = 0; l < 5; ++l) st(U + l * n3, ul[l]);
+    for (int l = 0; l < 5; ++l) P.put(U + l * n3, ul[l]);
     const T vx = ul[1] / ul[0], vy = ul[2] / ul[0], vz = ul[3] / ul[0];
     const T rho = ul[0] / rg;
     const T kin = rho * (vx * vx + vy * vy + vz * vz) / T(2);
@@ -331,7 +315,7 @@ __global__ __launch_bounds__(256) void k_tvd_flux(T* __restrict__ V, T* __restri
     const T blim2 = cs * sqrt(B2 * B2 + B4 * B4 + B5 * B5) + fabs(vv2);
     const T blim3 = cs * sqrt(B3 * B3 + B5 * B5 + B6 * B6) + fabs(vv3);
     cp = dmax(dmax(blim1, blim2), blim3);
-    st(c, cp);
+    P.put(c, cp);
   } else {
     cp = *(const T*)((const char*)(c + pl) + o);
   }
@@ -354,9 +338,9 @@ __global__ __launch_bounds__(256) void k_tvd_flux(T* __restrict__ V, T* __restri
     const T vtt1 = v1[0][l] - ulv * pdxg;
     const T vtt2 = v1[1][l] - ulv * pdyg;
     const T vtt3 = v1[2][l] - ulv * pdzg;
-    st(V + (0 * 5 + l) * n3, (b11 * vtt1 + b12 * vtt2 + b13 * vtt3) / cp);
-    st(V + (1 * 5 + l) * n3, (b12 * vtt1 + b22 * vtt2 + b23 * vtt3) / cp);
-    st(V + (2 * 5 + l) * n3, (b13 * vtt1 + b23 * vtt2 + b33 * vtt3) / cp);
+    P.put(V + (0 * 5 + l) * n3, (b11 * vtt1 + b12 * vtt2 + b13 * vtt3) / cp);
+    P.put(V + (1 * 5 + l) * n3, (b12 * vtt1 + b22 * vtt2 + b23 * vtt3) / cp);
+    P.put(V + (2 * 5 + l) * n3, (b13 * vtt1 + b23 * vtt2 + b33 * vtt3) / cp);
   }
 }
 
