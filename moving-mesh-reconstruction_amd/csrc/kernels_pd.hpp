@@ -109,7 +109,7 @@ struct PdSearch {
   const float4* xo;
   const unsigned* bits;
   const unsigned* near;  // bits_near, nwords per level
-  const int* out;        // whether any position lies outside [0, ng]: the search is k_pd_out's
+  const int* out;        // whether any position lies outside [0, ng]: the search is k_pd_far's alone
   i64 nwords;
   int ng, rmax;
 };
@@ -234,10 +234,21 @@ __global__ __launch_bounds__(256) void k_pd_nearest(int* __restrict__ near, int*
   for (int q = threadIdx.x; q < count; q += 256) far[1 + base + q] = list[q];
 }
 
-// Second pass, over far.
+// Second pass, over far; or, where positions lie outside [0, ng] or are NaN (at no distance: a cube that
+// holds no other particle does not end the search), the whole search.  A test beside the select in the search
+// loops cost k_pd_nearest 5 % (18 us at 200^3), a launch of its own 5 us.
 __global__ __launch_bounds__(256) void k_pd_far(int* __restrict__ near, int* __restrict__ wp, const int* __restrict__ far,
                                                 PdSearch P) {
-  if (*P.out) return;
+  if (*P.out) {
+    const unsigned ncell = (unsigned)P.ng * P.ng * P.ng;
+    for (unsigned c = blockIdx.x * 256u + threadIdx.x; c < ncell; c += gridDim.x * 256u) {
+      int best = -1;
+      if (P.end[c] <= P.start[c]) best = pd_search<false, true>(P, c, 1);
+      near[c] = best;
+      if (best >= 0) atomicAdd(&wp[best], 1);
+    }
+    return;
+  }
   const int count = far[0];
   for (int q = blockIdx.x * 256 + threadIdx.x; q < count; q += gridDim.x * 256) {
     const unsigned c = (unsigned)far[1 + q];
@@ -255,20 +266,6 @@ __global__ __launch_bounds__(256) void k_pd_far(int* __restrict__ near, int* __r
       }
     }
     const int best = pd_search<false>(P, c, r0);
-    near[c] = best;
-    if (best >= 0) atomicAdd(&wp[best], 1);
-  }
-}
-
-// The search where positions lie outside [0, ng] or are NaN (at no distance: a cube that holds no other
-// particle does not end the search), instead of both passes.  A test beside the select in their loops
-// cost k_pd_nearest 5 % (18 us at 200^3), the launch that ends at once 5 us.
-__global__ __launch_bounds__(256) void k_pd_out(int* __restrict__ near, int* __restrict__ wp, PdSearch P) {
-  if (!*P.out) return;
-  const unsigned ncell = (unsigned)P.ng * P.ng * P.ng;
-  for (unsigned c = blockIdx.x * 256u + threadIdx.x; c < ncell; c += gridDim.x * 256u) {
-    int best = -1;
-    if (P.end[c] <= P.start[c]) best = pd_search<false, true>(P, c, 1);
     near[c] = best;
     if (best >= 0) atomicAdd(&wp[best], 1);
   }

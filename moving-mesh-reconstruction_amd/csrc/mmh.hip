@@ -2592,7 +2592,6 @@ int mmh_particle_density_f(mmh_ctx* c, const float* xp, long long np, int ng, fl
     const int chunks = (int)std::min<i64>(PD_CH, std::max<i64>(1, ncell / 256 / 2048));
     k_pd_nearest<<<nblk(ncell, 256 * chunks), 256, 0, c->stream>>>(near, wp, far, P, chunks);
     k_pd_far<<<(unsigned)std::min<i64>(nblk(ncell), 8192), 256, 0, c->stream>>>(near, wp, far, P);
-    k_pd_out<<<(unsigned)std::min<i64>(nblk(ncell), 512), 256, 0, c->stream>>>(near, wp, P);
     k_pd_density<<<nblk(ncell), 256, 0, c->stream>>>(den, near, wp, start, end, order, ncell);
     LAUNCHCHK();
     double* sum = wsT<double>(c, "pd_sum", 1);
