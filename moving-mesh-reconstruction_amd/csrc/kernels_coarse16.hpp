@@ -16,9 +16,9 @@
 // and fifth colour of a sweep, and the last of a sweep with the first of the next, share a phase:
 // 6 phases per sweep instead of 8, the same values.
 // The per-point arithmetic, the order of every sum and the schedule are cw_cycle's, so results are
-// bit-identical.  Measured (MI355X), per cycle: FP32 reference schedule 1124 -> 244 us at NG = 64 and
-// 5.87 -> 1.22 ms at NG = 512 (0.24 us per phase); FP64 Krylov schedule with Galerkin levels 408 -> 127 us;
-// in a batch, one workgroup per grid, 614 -> 128 us.
+// bit-identical.  Measured (MI355X), per cycle: FP32 reference schedule 1124 -> 248 us at NG = 64 and
+// 5.87 -> 1.22 ms at NG = 512 (0.24 us per phase); FP64 Krylov schedule with Galerkin levels 408 -> 126 us;
+// in a batch, one workgroup per grid, 614 -> 129 us.
 #pragma once
 #include <limits>
 
@@ -34,9 +34,10 @@ namespace mmh {
 // 2^-80 and |b| up to 2^44 (FP64 2^-600, 2^400), make |q| large enough too.  A Range holds the
 // smallest dividend but zero of a thread, in two integer operations a quotient; where it or a divisor is out
 // of bounds, or the iterate is not finite (a quotient that overflows leaves it so), the cycle is run
-// again by the general form, whose divisions are plain.  A test on every quotient that chose the
-// division there cost 9 % of the FP32 cycle, flags of three comparisons 6 %.
-struct Range {
+// again with plain divisions.  A test on every quotient that chose the division there cost 9 % of
+// the FP32 cycle, flags of three comparisons 6 %.
+template <bool PLAIN> struct Range {
+  static constexpr bool plain = PLAIN;  // the cycle run again: plain divisions
   unsigned key = ~0u;  // of the smallest dividend: its bits without the sign, less one
   static __device__ __forceinline__ unsigned key_of(float a) { return (__float_as_uint(a) << 1) - 1u; }
   static __device__ __forceinline__ unsigned key_of(double a) {  // of the high word; one more below it if the low is set
@@ -62,11 +63,13 @@ __device__ __forceinline__ double corrected(double a, double b, double y, double
 }
 __device__ __forceinline__ float fixup(float q, float b, float a) { return __builtin_amdgcn_div_fixupf(q, b, a); }
 __device__ __forceinline__ double fixup(double q, double b, double a) { return __builtin_amdgcn_div_fixup(q, b, a); }
-template <class T> __device__ __forceinline__ T recip(T b, Range& off) {
+template <class T, class R> __device__ __forceinline__ T recip(T b, R& off) {
+  if constexpr (R::plain) return T(0);
   off.divisor(b);
   return T(1) / b;
 }
-template <class T> __device__ __forceinline__ T quotient(T a, T b, T y, Range& off) {
+template <class T, class R> __device__ __forceinline__ T quotient(T a, T b, T y, R& off) {
+  if constexpr (R::plain) return a / b;
   off.dividend(a);
   T q = a * y;
   q = corrected(a, b, y, q);
@@ -148,7 +151,7 @@ template <class T, int N> struct PointOp<T, N, false> {
   int nb[18];
   T w[7], x[12], y, b, b2;
   T di2;
-  __device__ __forceinline__ void load(const T* G, const T* rhs, int p, T dx, Range& off) {
+  template <class R> __device__ __forceinline__ void load(const T* G, const T* rhs, int p, T dx, R& off) {
     int i, j, k;
     point_of<1, true>(p, N, i, j, k);
 #pragma unroll
@@ -162,7 +165,7 @@ template <class T, int N> struct PointOp<T, N, false> {
     b2 = b * (dx * dx);
     di2 = T(1) / (dx * dx);
   }
-  __device__ __forceinline__ T update(const T* u, Range& off) const {
+  template <class R> __device__ __forceinline__ T update(const T* u, R& off) const {
     T q[18], t1, t2;
 #pragma unroll
     for (int e = 0; e < 18; ++e) q[e] = u[nb[e]];
@@ -181,7 +184,7 @@ template <class T, int N> struct PointOp<T, N, false> {
 template <class T, int N> struct PointOp<T, N, true> {
   int nb[27];
   T a[27], y, b;
-  __device__ __forceinline__ void load(const T* A, const T* rhs, int p, T, Range& off) {
+  template <class R> __device__ __forceinline__ void load(const T* A, const T* rhs, int p, T, R& off) {
     int i, j, k;
     point_of<1, true>(p, N, i, j, k);
 #pragma unroll
@@ -202,7 +205,7 @@ template <class T, int N> struct PointOp<T, N, true> {
       if (e != 13) s = s + a[e] * q[e];
     return s;
   }
-  __device__ __forceinline__ T update(const T* u, Range& off) const { return quotient(b - offsum(u), a[13], y, off); }
+  template <class R> __device__ __forceinline__ T update(const T* u, R& off) const { return quotient(b - offsum(u), a[13], y, off); }
   __device__ __forceinline__ T resid(const T* u, int p) const { return b - (offsum(u) + a[13] * u[p]); }
   template <class F> static __device__ __forceinline__ void phases(int ns, bool rev, F&& f) { phases27(ns, rev, f); }
 };
@@ -282,9 +285,9 @@ __device__ __forceinline__ void cc_zerosum(T* u, double* scal, int* guard, int m
 
 // The 4^3 level (cw_bottom), by wavefront 0: u4 holds the result.  Its mean's tree has one block of
 // which 64 threads hold a value, so the levels above h = 32 add zeros.
-template <class T, bool GAL>
+template <class T, bool GAL, class R>
 __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T dx, int nc, bool rev, double* scal, int* guard,
-                                          int ref, int mode, Range& off) {
+                                          int ref, int mode, R& off) {
   if (threadIdx.x >= 64) return;
   const int p = threadIdx.x;
   PointOp<T, 4, GAL> P;
@@ -314,9 +317,9 @@ __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T d
 
 // Sweeps of the 8^3 level; want: 0 none, 1 the residual into r8 (its maximum returned when norm), 2 the
 // maximum only.
-template <class T, bool GAL>
+template <class T, bool GAL, class R>
 __device__ __forceinline__ double cc_level8(T* u, const T* rhs, T* r8, const T* op, T dx, int ns, bool rev, int want, int norm,
-                                            Cc16Scratch& S, Range& off) {
+                                            Cc16Scratch& S, R& off) {
   const int p = threadIdx.x;
   PointOp<T, 8, GAL> P;
   P.load(op, rhs, p, dx, off);
@@ -368,9 +371,9 @@ template <int C = 0, class F> __device__ __forceinline__ void each_class(unsigne
 // 19-point: faces and the diagonal's reciprocal in registers; in FP32 the diagonal, the right-hand side and
 // the cross factors too; in FP64 (256 registers hold half as many values) the cross factors come from
 // G2, G3, G5 in LDS (big).
-template <class T>
+template <class T, class R>
 __device__ __forceinline__ double cc_level16_19(T* u, const T* rhs, T* r, T* big, const T* G, T dx, int ns, bool rev, int want,
-                                                int norm, Cc16Scratch& S, Range& off) {
+                                                int norm, Cc16Scratch& S, R& off) {
   constexpr bool REG = sizeof(T) == 4;
   const int q = threadIdx.x;
   Cell16 K;
@@ -474,9 +477,9 @@ constexpr int rank27(int e, int corner) {  // index of offset e among the corner
   for (int f = 0; f < e; ++f) r += corner27(f) == corner ? 1 : 0;
   return r;
 }
-template <class T>
+template <class T, class R>
 __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big, const T* A, int ns, bool rev, int want,
-                                                int norm, Cc16Scratch& S, Range& off) {
+                                                int norm, Cc16Scratch& S, R& off) {
   constexpr bool REG = sizeof(T) == 4;
   const int q = threadIdx.x;
   Cell16 K;
@@ -602,12 +605,12 @@ template <class P> __device__ __forceinline__ P* uniform(P* p) {
 
 // Levels C.n[0] (16, 8 or 4) .. 4 of the cycle C (cw_cycle's schedule), by CW threads, up to the entry
 // level's iterate, which is left in LDS; whether a quotient of this thread was out of range.
-template <class T> __device__ __forceinline__ bool cc16_levels(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
+template <class T, bool PLAIN> __device__ __forceinline__ bool cc16_levels(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
   static_assert(CW == 512, "one 16^3 cell, and one 8^3 point, per thread");
   const int t = threadIdx.x, lb = C.nl - 1, l8 = C.nl - 2, l16 = C.nl - 3;
   T* r16 = M.big;
-  Range off;   // of the levels in T
-  Range offd;  // of the FP64 4^3 level (mixed)
+  Range<PLAIN> off;   // of the levels in T
+  Range<PLAIN> offd;  // of the FP64 4^3 level (mixed)
   double r1_16 = 0.0, r1_8 = 0.0;
   // the entry level's iterate and right-hand side; coarser levels start from 0
   if (l16 >= 0) {
@@ -674,28 +677,11 @@ template <class T> __device__ __forceinline__ bool cc16_levels(const CoarseCycle
   return off.template out<T>() || offd.template out<double>();
 }
 
-// The general form (cw_cycle), called, not inlined: its registers and the level table's indexing would
-// otherwise cost the levels on chip spills.  Scratch and the level table are in LDS.
-template <class T> struct Cc16General {
-  double s[CW / RB][RB], blk[64], blk2[64], wm[CW / 64];
-  CoarseCycle<T> C;
-};
-template <class T> __device__ __attribute__((noinline)) void cc16_general(Cc16General<T>* g) {
-  cw_cycle<T>(g->C, g->s, g->blk, g->blk2, g->wm);
-}
-
-// The cycle; off the quotients' range by the general form, from the caller's arrays, which the levels on
-// chip have only read but for the per-level scalars and guards, formed again.
+// The cycle; off the quotients' range once more with plain divisions, from the caller's arrays, which the
+// levels on chip have only read but for the per-level scalars and guards, formed again.
 template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
   const int t = threadIdx.x;
-  if (__syncthreads_or(cc16_levels<T>(C, M))) {
-    static_assert(sizeof(Cc16General<T>) <= sizeof(M.big), "the general form's LDS lies in the staged coefficients'");
-    Cc16General<T>* g = reinterpret_cast<Cc16General<T>*>(M.big);
-    if (t == 0) g->C = C;
-    __syncthreads();
-    cc16_general<T>(g);
-    return;
-  }
+  if (__syncthreads_or(cc16_levels<T, false>(C, M))) cc16_levels<T, true>(C, M);
   if (C.nl == 1) {
     if (t < 64) C.u[0][t] = M.u4[t];
   } else if (C.nl == 2) {
