@@ -13,8 +13,8 @@
  *    completed.  _host entry points take host pointers and copy through context buffers.
  *  - Every entry point returns MMH_OK or an error code; nothing exits the process (the reference
  *    calls stop / pause, mmh/multigrid.f90:28-35,83-86, mmh/gauss1.f90:243-254).
- *  - N must be a power of two, 4 <= N <= 1024 for the solver (16 <= N for relaxing and the
- *    limiter, which the reference also requires, mmh/relaxing.f90:18).
+ *  - N must be a power of two, 4 <= N <= 1024 for the solver, smoothing and the spectral outputs (16 <= N for
+ *    relaxing and the limiter, which the reference also requires, mmh/relaxing.f90:18).
  */
 #ifndef MMH_H
 #define MMH_H
