@@ -16,9 +16,9 @@
 // and fifth colour of a sweep, and the last of a sweep with the first of the next, share a phase:
 // 6 phases per sweep instead of 8, the same values.
 // The per-point arithmetic, the order of every sum and the schedule are cw_cycle's, so results are
-// bit-identical.  Measured (MI355X), per cycle: FP32 reference schedule 1124 -> 248 us at NG = 64 and
+// bit-identical.  Measured (MI355X), per cycle: FP32 reference schedule 1124 -> 246 us at NG = 64 and
 // 5.87 -> 1.22 ms at NG = 512 (0.24 us per phase); FP64 Krylov schedule with Galerkin levels 408 -> 126 us;
-// in a batch, one workgroup per grid, 614 -> 129 us.
+// in a batch, one workgroup per grid, 614 -> 128 us.
 #pragma once
 #include <limits>
 
@@ -51,6 +51,7 @@ template <bool PLAIN> struct Range {
     if (!(fabs(b) >= 0x1p-1022 && fabs(b) <= 0x1p400)) key = 0u;
   }
   template <class T> __device__ __forceinline__ void iterate(T u) {
+    if constexpr (PLAIN) return;
     if (!(fabs(u) <= std::numeric_limits<T>::max())) key = 0u;
   }
   template <class T> __device__ __forceinline__ bool out() const { return key < key_of(sizeof(T) == 4 ? T(0x1p-80) : T(0x1p-600)); }
@@ -226,6 +227,7 @@ __device__ __forceinline__ double max64(double a) {
 struct Cc16Scratch {
   double s[CW];
   double v[CW / 64];
+  int off;  // a quotient was out of range (Range)
 };
 
 // max over the workgroup, in every thread.
@@ -285,11 +287,12 @@ __device__ __forceinline__ void cc_zerosum(T* u, double* scal, int* guard, int m
 
 // The 4^3 level (cw_bottom), by wavefront 0: u4 holds the result.  Its mean's tree has one block of
 // which 64 threads hold a value, so the levels above h = 32 add zeros.
-template <class T, bool GAL, class R>
+template <class T, bool GAL, bool PLAIN>
 __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T dx, int nc, bool rev, double* scal, int* guard,
-                                          int ref, int mode, R& off) {
+                                          int ref, int mode, Cc16Scratch& S) {
   if (threadIdx.x >= 64) return;
   const int p = threadIdx.x;
+  Range<PLAIN> off;
   PointOp<T, 4, GAL> P;
   P.load(op, rhs4, p, dx, off);
   auto phase = [&](unsigned mask) {
@@ -302,6 +305,7 @@ __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T d
   PointOp<T, 4, GAL>::phases(nc, rev, phase);
   if (ref) re = max64((double)fabs(P.resid(u4, p)));
   off.iterate(u4[p]);
+  if (off.template out<T>()) S.off = 1;
   double sum = tree64(0.0 + (double)u4[p]);
   sum = __shfl(sum, 0);
   bool g = false;
@@ -317,10 +321,11 @@ __device__ __forceinline__ void cc_bottom(T* u4, const T* rhs4, const T* op, T d
 
 // Sweeps of the 8^3 level; want: 0 none, 1 the residual into r8 (its maximum returned when norm), 2 the
 // maximum only.
-template <class T, bool GAL, class R>
+template <class T, bool GAL, bool PLAIN>
 __device__ __forceinline__ double cc_level8(T* u, const T* rhs, T* r8, const T* op, T dx, int ns, bool rev, int want, int norm,
-                                            Cc16Scratch& S, R& off) {
+                                            Cc16Scratch& S) {
   const int p = threadIdx.x;
+  Range<PLAIN> off;
   PointOp<T, 8, GAL> P;
   P.load(op, rhs, p, dx, off);
   const int cls = __builtin_amdgcn_readfirstlane(p >> 6);
@@ -329,6 +334,7 @@ __device__ __forceinline__ double cc_level8(T* u, const T* rhs, T* r8, const T* 
     __syncthreads();
   });
   off.iterate(u[p]);
+  if (off.template out<T>()) S.off = 1;
   if (!want) return 0.0;
   const T rv = P.resid(u, p);
   if (want == 1) r8[p] = rv;
@@ -371,13 +377,14 @@ template <int C = 0, class F> __device__ __forceinline__ void each_class(unsigne
 // 19-point: faces and the diagonal's reciprocal in registers; in FP32 the diagonal, the right-hand side and
 // the cross factors too; in FP64 (256 registers hold half as many values) the cross factors come from
 // G2, G3, G5 in LDS (big).
-template <class T, class R>
+template <class T, bool PLAIN>
 __device__ __forceinline__ double cc_level16_19(T* u, const T* rhs, T* r, T* big, const T* G, T dx, int ns, bool rev, int want,
-                                                int norm, Cc16Scratch& S, R& off) {
+                                                int norm, Cc16Scratch& S) {
   constexpr bool REG = sizeof(T) == 4;
   const int q = threadIdx.x;
   Cell16 K;
   K.set(q);
+  Range<PLAIN> off;
   T w[8][REG ? 7 : 6], y[8], b2[REG ? 8 : 1], x[REG ? 8 : 1][12];
   if constexpr (!REG) {
     for (int t = q; t < 4096; t += CW) {
@@ -449,6 +456,7 @@ __device__ __forceinline__ double cc_level16_19(T* u, const T* rhs, T* r, T* big
   });
 #pragma unroll
   for (int c = 0; c < 8; ++c) off.iterate(u[c * 512 + q]);
+  if (off.template out<T>()) S.off = 1;
   if (!want) return 0.0;
   const T di2 = T(1) / dx2;
   T rv[8];
@@ -477,9 +485,9 @@ constexpr int rank27(int e, int corner) {  // index of offset e among the corner
   for (int f = 0; f < e; ++f) r += corner27(f) == corner ? 1 : 0;
   return r;
 }
-template <class T, class R>
+template <class T, bool PLAIN>
 __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big, const T* A, int ns, bool rev, int want,
-                                                int norm, Cc16Scratch& S, R& off) {
+                                                int norm, Cc16Scratch& S) {
   constexpr bool REG = sizeof(T) == 4;
   const int q = threadIdx.x;
   Cell16 K;
@@ -487,6 +495,7 @@ __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big
   T rv[8];
   double am = 0.0;
   if constexpr (REG) {
+    Range<PLAIN> off;
     T a[8][19], y[8], b[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
@@ -519,6 +528,7 @@ __device__ __forceinline__ double cc_level16_27(T* u, const T* rhs, T* r, T* big
     });
 #pragma unroll
     for (int c = 0; c < 8; ++c) off.iterate(u[c * 512 + q]);
+    if (off.template out<T>()) S.off = 1;
     if (!want) return 0.0;
     each_class(0xFFu, [&](auto cc) {
       constexpr int c = decltype(cc)::value;
@@ -604,13 +614,11 @@ template <class P> __device__ __forceinline__ P* uniform(P* p) {
 }
 
 // Levels C.n[0] (16, 8 or 4) .. 4 of the cycle C (cw_cycle's schedule), by CW threads, up to the entry
-// level's iterate, which is left in LDS; whether a quotient of this thread was out of range.
-template <class T, bool PLAIN> __device__ __forceinline__ bool cc16_levels(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
+// level's iterate, which is left in LDS; M.S.off is set where a quotient was out of range.
+template <class T, bool PLAIN> __device__ __forceinline__ void cc16_levels(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
   static_assert(CW == 512, "one 16^3 cell, and one 8^3 point, per thread");
   const int t = threadIdx.x, lb = C.nl - 1, l8 = C.nl - 2, l16 = C.nl - 3;
   T* r16 = M.big;
-  Range<PLAIN> off;   // of the levels in T
-  Range<PLAIN> offd;  // of the FP64 4^3 level (mixed)
   double r1_16 = 0.0, r1_8 = 0.0;
   // the entry level's iterate and right-hand side; coarser levels start from 0
   if (l16 >= 0) {
@@ -625,8 +633,8 @@ template <class T, bool PLAIN> __device__ __forceinline__ bool cc16_levels(const
   }
   __syncthreads();
   if (l16 >= 0) {
-    if (C.A[l16]) r1_16 = cc_level16_27<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], false, 1, C.ref, M.S, off);
-    else r1_16 = cc_level16_19<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], false, 1, C.ref, M.S, off);
+    if (C.A[l16]) r1_16 = cc_level16_27<T, PLAIN>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], false, 1, C.ref, M.S);
+    else r1_16 = cc_level16_19<T, PLAIN>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], false, 1, C.ref, M.S);
     if (C.ref && t == 0) C.scal[l16][0] = r1_16;
     __syncthreads();
     restrict_point<T, 1, true>(M.rhs8, r16, 16, relax_plane(C.sw[l16], 16), t);
@@ -634,8 +642,8 @@ template <class T, bool PLAIN> __device__ __forceinline__ bool cc16_levels(const
     __syncthreads();
   }
   if (l8 >= 0) {
-    if (C.A[l8]) r1_8 = cc_level8<T, true>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S, off);
-    else r1_8 = cc_level8<T, false>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S, off);
+    if (C.A[l8]) r1_8 = cc_level8<T, true, PLAIN>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S);
+    else r1_8 = cc_level8<T, false, PLAIN>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], false, 1, C.ref, M.S);
     if (C.ref && t == 0) C.scal[l8][0] = r1_8;
     __syncthreads();
     if (t < 64) {
@@ -651,37 +659,39 @@ template <class T, bool PLAIN> __device__ __forceinline__ bool cc16_levels(const
       M.du[t] = 0.0;
     }
     __syncthreads();
-    if (C.dA) cc_bottom<double, true>(M.du, M.drhs, C.dA, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b, offd);
-    else cc_bottom<double, false>(M.du, M.drhs, C.dG, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b, offd);
+    if (C.dA) cc_bottom<double, true, PLAIN>(M.du, M.drhs, C.dA, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b, M.S);
+    else cc_bottom<double, false, PLAIN>(M.du, M.drhs, C.dG, C.ddx, C.coarse, C.symmetric, C.dscal, C.dguard, C.ref, mode_b, M.S);
     if (t < 64) M.u4[t] = (T)M.du[t];
   } else {
-    if (C.A[lb]) cc_bottom<T, true>(M.u4, M.rhs4, C.A[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b, off);
-    else cc_bottom<T, false>(M.u4, M.rhs4, C.G[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b, off);
+    if (C.A[lb]) cc_bottom<T, true, PLAIN>(M.u4, M.rhs4, C.A[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b, M.S);
+    else cc_bottom<T, false, PLAIN>(M.u4, M.rhs4, C.G[lb], C.dx[lb], C.coarse, C.symmetric, C.scal[lb], C.guard[lb], C.ref, mode_b, M.S);
   }
   __syncthreads();
-  if (l8 < 0) return off.template out<T>() || offd.template out<double>();
+  if (l8 < 0) return;
   if (t < 64) prolong_cell<T, true>(M.u8, M.u4, 8, 1, t);
   __syncthreads();
   double re;
-  if (C.A[l8]) re = cc_level8<T, true>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
-  else re = cc_level8<T, false>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
+  if (C.A[l8]) re = cc_level8<T, true, PLAIN>(M.u8, M.rhs8, M.r8, C.A[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
+  else re = cc_level8<T, false, PLAIN>(M.u8, M.rhs8, M.r8, C.G[l8], C.dx[l8], C.sw[l8], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
   if (C.ref && t == 0) C.scal[l8][1] = re;
   cc_zerosum<T, 8>(M.u8, C.scal[l8], C.guard[l8], (C.ref && !(C.top && l8 == 0)) ? 1 : 0, r1_8, re, M.S);
-  if (l16 < 0) return off.template out<T>() || offd.template out<double>();
+  if (l16 < 0) return;
   prolong_cell<T, true>(M.u16, M.u8, 16, 1, t);
   __syncthreads();
-  if (C.A[l16]) re = cc_level16_27<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
-  else re = cc_level16_19<T>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S, off);
+  if (C.A[l16]) re = cc_level16_27<T, PLAIN>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.A[l16]), C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
+  else re = cc_level16_19<T, PLAIN>(M.u16, uniform(C.rhs[l16]), r16, M.big, uniform(C.G[l16]), C.dx[l16], C.sw[l16], C.symmetric != 0, C.ref ? 2 : 0, C.ref, M.S);
   if (C.ref && t == 0) C.scal[l16][1] = re;
   cc_zerosum<T, 16>(M.u16, C.scal[l16], C.guard[l16], (C.ref && !(C.top && l16 == 0)) ? 1 : 0, r1_16, re, M.S);
-  return off.template out<T>() || offd.template out<double>();
 }
 
 // The cycle; off the quotients' range once more with plain divisions, from the caller's arrays, which the
 // levels on chip have only read but for the per-level scalars and guards, formed again.
 template <class T> __device__ __forceinline__ void cc16_cycle(const CoarseCycle<T>& C, Cc16Lds<T>& M) {
   const int t = threadIdx.x;
-  if (__syncthreads_or(cc16_levels<T, false>(C, M))) cc16_levels<T, true>(C, M);
+  if (t == 0) M.S.off = 0;  // every level starts behind a barrier
+  cc16_levels<T, false>(C, M);
+  __syncthreads();
+  if (M.S.off) cc16_levels<T, true>(C, M);
   if (C.nl == 1) {
     if (t < 64) C.u[0][t] = M.u4[t];
   } else if (C.nl == 2) {
